@@ -347,6 +347,18 @@ int vrm_turboquant_compress(const void* kv, int src_dtype, int N, int head_dim,
                             uint16_t* radius, uint8_t* angles, uint8_t* qjl_signs,
                             uint16_t* qjl_norms, vrm_stream_t stream);
 
+/* The same codes in the packed format (vrm_pack_bits of the angles with `bits`
+ * and of the signs with 1 bit): angles_packed [N][((padded_dim - 1) bits + 7) / 8],
+ * signs_packed [N][qjl_dim / 8], both aligned to 4 bytes.  Serves padded_dim 64
+ * or 128, 2 to 4 bits and qjl_dim = padded_dim / 2; VRM_ERR_UNSUPPORTED
+ * otherwise (compress, then vrm_pack_bits). */
+int vrm_turboquant_compress_packed(const void* kv, int src_dtype, int N, int head_dim,
+                                   int padded_dim, int n_levels, int bits, int qjl_dim,
+                                   const float* signs, const float* jl, const float* angle_lut,
+                                   uint16_t* radius, uint8_t* angles_packed,
+                                   uint8_t* signs_packed, uint16_t* qjl_norms,
+                                   vrm_stream_t stream);
+
 /*
  * out[N][head_dim] float32 = unrotate(polar_decode(radius, angles)), no QJL
  * (core/kv_quantizer.py:481-500).  Replaces the pybind entry `decompress` of

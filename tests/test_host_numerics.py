@@ -19,6 +19,7 @@ CSRC = os.path.join(ROOT, "vramancer_amd", "csrc")
 SRC = r"""
 #include "vrm_fdlibm_atan2f.h"
 #include "vrm_e4m3.h"
+#include "vrm_tq_bin.h"
 #include <math.h>
 #include <stdint.h>
 extern "C" long atan2_mismatches(long n, uint64_t seed, int mode) {
@@ -36,6 +37,59 @@ extern "C" long atan2_mismatches(long n, uint64_t seed, int mode) {
     }
     float a = vrm_fdlibm::atan2f(y, x), b = ::atan2f(y, x);
     if (vrm_fdlibm::fbits(a) != vrm_fdlibm::fbits(b) && !(isnan(a) && isnan(b))) ++bad;
+  }
+  return bad;
+}
+// bins off the sector edges that differ from the defining atan2; values drawn
+// over 80 binary orders, at ratios within 2^-19 of 1 and within 1e-5 rad of an edge
+template <int BITS, bool L0> static long bins(long n, uint64_t seed, long* edges) {
+  uint64_t s = seed * 6364136223846793005ull + 1442695040888963407ull;
+  auto next = [&]() { s ^= s << 13; s ^= s >> 7; s ^= s << 17; return s; };
+  auto uni = [&]() { return (double)(next() >> 11) / 9007199254740992.0; };
+  const float lo0 = (float)-3.141592653589793, r0 = (float)6.283185307179586, r1 = (float)1.5707963267948966;
+  long bad = 0;
+  for (long i = 0; i < n; ++i) {
+    float x = (float)(4 * uni() - 2), y = (float)(4 * uni() - 2);
+    if (i % 4 == 1) y = x * (1.0f + ldexpf((float)((int)(next() % 65) - 32), -24));
+    if (i % 4 == 2) {
+      const double step = (L0 ? 2 * M_PI : M_PI / 2) / (1 << BITS);
+      const double th = (L0 ? -M_PI : 0.0) + step * (double)(next() % ((1 << BITS) + 1)) + (uni() - 0.5) * 2e-5;
+      const double r = 0.01 + uni();
+      x = (float)(r * cos(th)); y = (float)(r * sin(th));
+    }
+    if (i % 4 == 3) { x = ldexpf(x, -(int)(next() % 40)); y = ldexpf(y, -(int)(next() % 40)); }
+    if (!L0) { x = fabsf(x); y = fabsf(y); }
+    // the reciprocal off by up to one ulp either way
+    const float rcp = vrm_fdlibm::bitsf(vrm_fdlibm::fbits(1.0f / fmaxf(fabsf(x), fabsf(y))) + (uint32_t)(next() % 3) - 1u);
+    bool edge;
+    const int got = vrm_tq_bin::fast_bin<BITS, L0>(x, y, rcp, edge);
+    if (edge) { ++*edges; continue; }
+    const float th = vrm_fdlibm::atan2f(y, x);
+    const float d = th - lo0;
+    const float nrm = L0 ? d / r0 : th / r1;
+    const float t = nrm * (float)(1 << BITS);
+    int ref = (int)t;
+    ref = ref < 0 ? 0 : ref > (1 << BITS) - 1 ? (1 << BITS) - 1 : ref;
+    if (got != ref) ++bad;
+  }
+  return bad;
+}
+extern "C" long fast_bin_mismatches(int bits, int level0, long n, uint64_t seed, long* edges) {
+  switch (2 * bits + level0) {
+    case 4: return bins<2, false>(n, seed, edges);
+    case 5: return bins<2, true>(n, seed, edges);
+    case 6: return bins<3, false>(n, seed, edges);
+    case 7: return bins<3, true>(n, seed, edges);
+    case 8: return bins<4, false>(n, seed, edges);
+    default: return bins<4, true>(n, seed, edges);
+  }
+}
+extern "C" long div_sqrt128_mismatches(int exponent) {
+  const volatile float root = (float)sqrt(128.0);
+  long bad = 0;
+  for (uint32_t m = 0; m < (1u << 23); ++m) {
+    const float x = vrm_fdlibm::bitsf(((uint32_t)(exponent + 127) << 23) | m);
+    if (x / root != vrm_tq_bin::div_sqrt128(x)) ++bad;
   }
   return bad;
 }
@@ -84,6 +138,25 @@ def test_fdlibm_atan2f_special_values(hostlib):
         for x in sp:
             a, b = hostlib.atan2_one(y, x), libm.atan2f(y, x)
             assert np.float32(a).view(np.uint32) == np.float32(b).view(np.uint32), (y, x)
+
+
+@pytest.mark.parametrize("level0", [0, 1])
+@pytest.mark.parametrize("bits", [2, 3, 4])
+def test_fast_bin_is_the_defined_bin_off_the_edges(hostlib, bits, level0):
+    edges = ctypes.c_long(0)
+    hostlib.fast_bin_mismatches.restype = ctypes.c_long
+    hostlib.fast_bin_mismatches.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_long, ctypes.c_uint64, ctypes.c_void_p]
+    n = 2_000_000
+    assert hostlib.fast_bin_mismatches(bits, level0, n, 7 + bits, ctypes.byref(edges)) == 0
+    # the ordinary quarter of the draws is hardly ever at an edge
+    assert edges.value < 0.76 * n
+
+
+@pytest.mark.parametrize("exponent", [-100, -3, 0, 1, 100])
+def test_div_sqrt128_is_correctly_rounded(hostlib, exponent):
+    # every significand of a binary order; the operation is the same in each
+    hostlib.div_sqrt128_mismatches.restype = ctypes.c_long
+    assert hostlib.div_sqrt128_mismatches(exponent) == 0
 
 
 def test_e4m3_encode_matches_torch_cast(hostlib):

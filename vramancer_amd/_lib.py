@@ -58,6 +58,7 @@ SIGNATURES = {
     "vrm_kv_quant_pages": (_i, [_p, _p, _i, _p, _p, _i, _p, _p, _i] + [_i] * 6 + [_p]),
     "vrm_kv_dequant_pages": (_i, [_p, _p, _i, _p, _i, _p] + [_i] * 6 + [_p]),
     "vrm_turboquant_compress": (_i, [_p, _i, _i, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p]),
+    "vrm_turboquant_compress_packed": (_i, [_p, _i, _i, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p]),
     "vrm_turboquant_decompress": (_i, [_p, _p, _i, _i, _i, _i, _i, _p, _p, _p, _i, _p]),
     "vrm_tq_slice_bytes": (_sz, [_i, _i, _i]),
     "vrm_tq_slice_bytes_ps": (_sz, [_i, _i, _i, _i]),

@@ -17,11 +17,13 @@
 //            BLAS order is unknown; ties within its rounding are documented);
 //            norm with eight interleaved fused accumulators summed in order,
 //            which is how PyTorch's CPU 2-norm kernel reduces a 128-float row.
-// One 64-lane wavefront per row; the row lives in LDS between stages.
+// One 64-lane wavefront per row; the row lives in LDS between stages.  Calls of
+// many rows at the common settings go to the tile encoder (vrm_tq_encode.hip).
 #include "vrm_common.h"
-#include "vrm_fdlibm_atan2f.h"
 #include "vrm_tq_common.h"
+#include "vrm_tq_encode.h"
 #include "vrm_tq_layout.h"
+#include "vrm_tq_row.h"
 
 #include <math.h>
 
@@ -43,173 +45,22 @@ struct TqArgs {
   float* out;        // decompress output
 };
 
-// Element e of the polar decode of one row from the fp32 radius and the
-// level-major bins (level l at offset PD - (PD >> l)).  The reference decodes
-// level by level from the top, each value r of level l becoming the pair
-// (r cos, r sin) of level l - 1; element e is therefore the product chain
-//   ((radius * f_{NL-1}) * f_{NL-2}) ... * f_0,
-// f_l the cos (bit l of e clear) or sin (set) of angle e >> (l + 1) of level
-// l, the same roundings in the same order, with no exchange between lanes.
-template <int PD>
-__device__ __forceinline__ float polar_element(float radius, const uint8_t* bins, const float* lut, int nb, int e) {
-  constexpr int NL = __builtin_ctz(PD);
-  float r = radius;
-#pragma unroll
-  for (int l = NL - 1; l >= 0; --l) {
-    const int idx = min((int)bins[PD - (PD >> l) + (e >> (l + 1))], nb - 1);  // caller-supplied bins stay in the table
-    r = __fmul_rn(r, lut[(l == 0 ? 0 : 2 * nb) + (((e >> l) & 1) ? nb : 0) + idx]);
-  }
-  return r;
-}
-
-// Polar decode of one row into `recon` (LDS, PD floats); bins may have been
-// written by any lane before the call, recon is visible to every lane after.
-template <int PD>
-__device__ __forceinline__ void polar_decode(float radius, const uint8_t* bins, const float* lut, int nb,
-                                             float* recon, int lane) {
-  row_sync();
-#pragma unroll
-  for (int k = 0; k < tq_per_lane(PD); ++k)
-    if (k * 64 + lane < PD) recon[k * 64 + lane] = polar_element<PD>(radius, bins, lut, nb, k * 64 + lane);
-  row_sync();
-}
-
-// LDS working set of one row.
-template <int PD>
-struct RowLds {
-  float rot[PD];               // rotated row
-  float rad[PD];               // radius of each polar node, level-major like the bins
-  alignas(16) double res[PD];  // QJL residual, widened once by the lane that owns it
-  uint8_t bins[PD];
-  float norm_acc[8];
-};
-
-// Rotation and polar encoding of one row (source element e at src[e] for
-// e < head_dim, zero padding above): leaves the level-major bins in w.bins,
-// the rotated row in v (element e in lane e % 64, register e / 64; lanes past
-// a row of fewer than 64 elements hold zeros) and in w.rot, and returns the
-// fp32 final radius.
-template <int SRC, int PD>
-__device__ __forceinline__ float encode_row(const void* src, size_t first, int head_dim, const float* signs, int bits,
-                                            float (&v)[tq_per_lane(PD)], RowLds<PD>& w, int lane) {
-  constexpr int PER = tq_per_lane(PD);
-  constexpr int NL = __builtin_ctz(PD);
-  const int nb = 1 << bits;
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const int e = k * 64 + lane;
-    const float x = e < head_dim ? load_row<SRC>(src, first + e) : 0.f;
-    v[k] = e < PD ? __fmul_rn(x, signs[e]) : 0.f;
-  }
-  fwht<PD>(v, lane);
-  const float root = (float)sqrt((double)PD);
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    v[k] = __fdiv_rn(v[k], root);
-    if (k * 64 + lane < PD) w.rot[k * 64 + lane] = v[k];
-  }
-  row_sync();
-
-  // The radii only need square roots, level after level: node i of level l
-  // (w.rad[PD - (PD >> l) + i]) over children 2 i, 2 i + 1 of level l - 1
-  // (the rotated row below level 0).
-  for (int level = 0; level < NL; ++level) {
-    const float* child = level == 0 ? w.rot : w.rad + (PD - (PD >> (level - 1)));
-    float* rad = w.rad + (PD - (PD >> level));
-    for (int i = lane; i < (PD >> (level + 1)); i += 64) {
-      const float x0 = child[2 * i], x1 = child[2 * i + 1];
-      rad[i] = sqrt_rn(__fadd_rn(__fadd_rn(__fmul_rn(x0, x0), __fmul_rn(x1, x1)), 1e-12f));
-    }
-    row_sync();
-  }
-  // With every child known, the angles of all levels are independent: lane
-  // takes bins b = lane, lane + 64, ... of the level-major order.
-  const float lo0 = (float)-3.141592653589793, range0 = (float)6.283185307179586;
-  const float range1 = (float)1.5707963267948966;
-  const float nbf = (float)nb;
-  for (int b = lane; b < PD - 1; b += 64) {
-    const int level = NL - 1 - (31 - __builtin_clz(PD - b - 1));  // PD >> (level + 1) < PD - b <= PD >> level
-    const int i = b - (PD - (PD >> level));
-    const float* child = level == 0 ? w.rot : w.rad + (PD - (PD >> (level - 1)));
-    const float x0 = child[2 * i], x1 = child[2 * i + 1];
-    const float th = vrm_fdlibm::atan2f(x1, x0);
-    const float nrm = level == 0 ? __fdiv_rn(__fsub_rn(th, lo0), range0) : __fdiv_rn(th, range1);
-    int idx = (int)__fmul_rn(nrm, nbf);  // truncation toward zero, as .long()
-    idx = min(max(idx, 0), nb - 1);
-    w.bins[b] = (uint8_t)idx;
-  }
-  row_sync();
-  return w.rad[PD - 2];
-}
-
-// Residual against the reconstruction from the fp32 radius, its QJL signs
-// (float64 dot products; sign(j) is handed to put_sign) and the residual norm
-// as PyTorch's CPU 2-norm reduces a row: eight interleaved fused accumulators
-// summed in order for rows of 4 floats or more, one fused chain for a row of
-// 2 (measured against torch.norm at 2 .. 256 floats).  Returns the norm.
-template <int PD, typename PutSign>
-__device__ __forceinline__ float qjl_row(const float (&v)[tq_per_lane(PD)], float radius, const float* lut, int bits,
-                                         const float* jl, int qjl_dim, RowLds<PD>& w, int lane, PutSign put_sign) {
-  constexpr int PER = tq_per_lane(PD);
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const int e = k * 64 + lane;
-    if (e < PD) w.res[e] = (double)__fsub_rn(v[k], polar_element<PD>(radius, w.bins, lut, 1 << bits, e));
-  }
-  row_sync();
-  // Lane j walks row j of the JL matrix.  With a 16-byte aligned matrix (every
-  // row is then aligned, PD being a multiple of 4) it reads four floats per
-  // load; the residual comes as doubles, two per LDS broadcast.  The
-  // accumulation order is the element order either way.
-  const bool vec = PD >= 4 && (reinterpret_cast<uintptr_t>(jl) & 15) == 0;
-  const double2* r2 = reinterpret_cast<const double2*>(w.res);
-  for (int j = lane; j < qjl_dim; j += 64) {
-    const float* jr = jl + (size_t)j * PD;
-    double s = 0.0;
-    if (vec) {
-      const float4* jr4 = reinterpret_cast<const float4*>(jr);
-#pragma unroll 8
-      for (int m = 0; m < PD / 4; ++m) {
-        const float4 x = jr4[m];
-        const double2 ra = r2[2 * m], rb = r2[2 * m + 1];
-        s = fma(ra.x, (double)x.x, s);
-        s = fma(ra.y, (double)x.y, s);
-        s = fma(rb.x, (double)x.z, s);
-        s = fma(rb.y, (double)x.w, s);
-      }
-    } else {
-      for (int e = 0; e < PD; ++e) s = fma(w.res[e], (double)jr[e], s);
-    }
-    put_sign(j, s > 0.0);
-  }
-  if constexpr (PD == 2) {
-    const float x0 = (float)w.res[0], x1 = (float)w.res[1];  // exact: widened from floats
-    return sqrt_rn(fmaf(x1, x1, __fmul_rn(x0, x0)));
-  }
-  if (lane < 8) {
-    float acc = 0.f;
-#pragma unroll
-    for (int m = 0; m < (PD + 7) / 8; ++m) {
-      if (lane + 8 * m < PD) {
-        const float x = (float)w.res[lane + 8 * m];  // exact: widened from a float
-        acc = fmaf(x, x, acc);
-      }
-    }
-    w.norm_acc[lane] = acc;
-  }
-  row_sync();
-  float s = w.norm_acc[0];
-#pragma unroll
-  for (int k = 1; k < 8; ++k) s = __fadd_rn(s, w.norm_acc[k]);
-  return sqrt_rn(s);
-}
-
 // Launch shape of the row kernels: a launch of at least kBulkMinRows rows
 // packs kBulkRows rows (one wavefront each) per workgroup, so a compute unit
 // holds more rows at once than its workgroup slots allow at one row each;
 // smaller launches keep one row per workgroup, spread over more units.
 constexpr int kBulkRows = 4;
 constexpr int kBulkMinRows = 4096;
+// Rows (of one K/V side) from which the tile encoder (vrm_tq_encode.hip) takes
+// over from one row per wavefront: below it the row kernels fill the chip with
+// more, shorter wavefronts.  Measured at 3 bits, row kernel / tile encoder:
+// padded dim 128 codec 1024 rows 10.0 / 14.5 us, 2048 13.4 / 13.3, 4096 20.1 /
+// 14.4, 65,536 236 / 28.4; pages 2 x 1536 rows 13.9 / 15.9 us, 2 x 2048 15.5 /
+// 13.8, 2 x 4096 29.2 / 13.9; padded dim 64 codec 1024 rows 6.3 / 7.7 us, 2048
+// 7.1 / 7.0, 65,536 84 / 15.3.  Pages at padded dim 64 are faster tiled at any
+// size (2 x 8 rows 7.1 / 6.4 us, 2 x 4096 16.7 / 8.1).
+constexpr int kTileMinRows = 2048;
+constexpr int kTileMaxRows = 0x7fffff00;
 
 // LUT_LDS: the angle table (4 x 2^bits floats, bits <= 4) is read from LDS.
 template <int SRC, int PD, int ROWS, bool LUT_LDS>
@@ -225,7 +76,9 @@ __global__ void __launch_bounds__(64 * ROWS) tq_compress_kernel(TqArgs a) {
   if (row >= a.N) return;
   RowLds<PD>& w = rows_lds[threadIdx.x >> 6];
   float v[tq_per_lane(PD)];
-  const float radius = encode_row<SRC, PD>(a.kv, (size_t)row * a.head_dim, a.head_dim, a.signs, a.bits, v, w, lane);
+  const size_t first = (size_t)row * a.head_dim;
+  const float radius = encode_row<PD>([&](int e) { return load_row<SRC>(a.kv, first + e); }, a.head_dim, a.signs,
+                                      a.bits, v, w, lane);
   for (int i = lane; i < PD - 1; i += 64) a.angles[(size_t)row * (PD - 1) + i] = w.bins[i];
   if (lane == 0) a.radius[row] = f32_to_f16_bits(radius);
   const float* lut = LUT_LDS ? lut_lds : a.lut;
@@ -239,7 +92,8 @@ __global__ void __launch_bounds__(64 * ROWS) tq_compress_kernel(TqArgs a) {
 // Writes TurboQuant codes straight into the pages of a TurboQuant pool
 // (layout in vrm_tq_layout.h).  One wavefront per (row, K/V): the codes are
 // those of tq_compress_kernel; V rows skip the QJL stage, whose output the
-// attention never reads for values.
+// attention never reads for values.  Serves the writes of few rows at padded
+// dim 128; vrm_tq_encode.hip the others.
 // ---------------------------------------------------------------------------
 struct TqPoolArgs {
   const void* key;
@@ -256,21 +110,19 @@ struct TqPoolArgs {
   const float* lut;
 };
 
-template <int SRC, int BITS, int ROWS, int PD>
-__global__ void __launch_bounds__(64 * ROWS) tq_pool_write_kernel(TqPoolArgs a) {
+template <int SRC, int BITS>
+__global__ void __launch_bounds__(64) tq_pool_write_kernel(TqPoolArgs a) {
   namespace L = vrm::tq;
+  constexpr int PD = 128;
   constexpr int QJL = L::tuned_qjl(PD);
   constexpr int SLICE = L::slice_bytes(PD, BITS);
-  __shared__ RowLds<PD> rows_lds[ROWS];
-  __shared__ uint32_t rows_signs[ROWS][QJL / 32];
+  __shared__ RowLds<PD> w;
+  __shared__ uint32_t sign_bits[QJL / 32];
   __shared__ float lut_lds[4 << BITS];  // the angle table ({level 0, levels >= 1} x {cos, sin} x 2^BITS)
-  const int lane = threadIdx.x & 63;
-  if (threadIdx.x < (4 << BITS)) lut_lds[threadIdx.x] = a.lut[threadIdx.x];
-  __syncthreads();  // the workgroup's only barrier, before any wavefront leaves
-  const int x = blockIdx.x * ROWS + (int)(threadIdx.x >> 6);
-  if (x >= a.rows) return;
-  RowLds<PD>& w = rows_lds[threadIdx.x >> 6];
-  uint32_t* sign_bits = rows_signs[threadIdx.x >> 6];
+  const int lane = threadIdx.x;
+  if (lane < (4 << BITS)) lut_lds[lane] = a.lut[lane];
+  __syncthreads();
+  const int x = blockIdx.x;
   const int kv = blockIdx.y;
   // append: x = n * KH + h (token n); pages: x = (np * KH + h) * 16 + t
   int n, h, t;
@@ -307,7 +159,8 @@ __global__ void __launch_bounds__(64 * ROWS) tq_pool_write_kernel(TqPoolArgs a) 
   }
   float v[tq_per_lane(PD)];
   const void* src = kv ? a.value : a.key;
-  const float radius = encode_row<SRC, PD>(src, src_first, a.head_dim, a.signs, BITS, v, w, lane);
+  const float radius = encode_row<PD>([&](int e) { return load_row<SRC>(src, src_first + e); }, a.head_dim, a.signs,
+                                      BITS, v, w, lane);
   // angle record: the PD slots (4 quarters of PD / 4) as one bit stream, so
   // dword k covers slots from the one holding bit 32 k, at most 32 / BITS + 2
   if (lane < abytes / 4) {
@@ -379,7 +232,8 @@ __global__ void __launch_bounds__(64) tq_pool_write_gen_kernel(TqPoolArgs a, tq:
   }
   float v[tq_per_lane(PD)];
   const void* src = kv ? a.value : a.key;
-  const float radius = encode_row<SRC, PD>(src, src_first, a.head_dim, a.signs, g.bits, v, w, lane);
+  const float radius = encode_row<PD>([&](int e) { return load_row<SRC>(src, src_first + e); }, a.head_dim, a.signs,
+                                      g.bits, v, w, lane);
   // angle dword k covers record bits [32 k, 32 k + 32): bins from the one holding bit 32 k
   for (int k = lane; k < g.angle_dw; k += 64) {
     uint32_t word = 0;
@@ -807,11 +661,10 @@ int check_tq(int N, int head_dim, int padded_dim, int n_levels, int bits, const 
 
 using namespace vrm;
 
-extern "C" int vrm_turboquant_compress(const void* kv, int src_dtype, int N, int head_dim, int padded_dim,
-                                       int n_levels, int bits, int qjl_dim, const float* signs, const float* jl,
-                                       const float* angle_lut, uint16_t* radius, uint8_t* angles,
-                                       uint8_t* qjl_signs, uint16_t* qjl_norms, vrm_stream_t stream) {
-  const char* who = "vrm_turboquant_compress";
+namespace {
+int check_compress(const void* kv, int src_dtype, int N, int head_dim, int padded_dim, int n_levels, int bits,
+                   int qjl_dim, const float* signs, const float* jl, const float* angle_lut, const void* radius,
+                   const void* angles, const void* qjl_signs, const void* qjl_norms, const char* who) {
   int rc = check_tq(N, head_dim, padded_dim, n_levels, bits, who);
   if (rc) return rc;
   if (qjl_dim <= 0 || qjl_dim > 4 * padded_dim) {
@@ -822,10 +675,49 @@ extern "C" int vrm_turboquant_compress(const void* kv, int src_dtype, int N, int
     set_error("%s: unknown source dtype %d", who, src_dtype);
     return VRM_ERR_ARG;
   }
-  if (N == 0) return VRM_OK;
-  if (!kv || !signs || !jl || !angle_lut || !radius || !angles || !qjl_signs || !qjl_norms) {
+  if (N > 0 && (!kv || !signs || !jl || !angle_lut || !radius || !angles || !qjl_signs || !qjl_norms)) {
     set_error("%s: null pointer argument", who);
     return VRM_ERR_ARG;
+  }
+  return VRM_OK;
+}
+
+TqEncodeArgs codec_args(const void* kv, int src_dtype, int N, int head_dim, int padded_dim, int bits, bool packed,
+                        const float* signs, const float* jl, const float* angle_lut, uint16_t* radius,
+                        uint8_t* angles, uint8_t* qjl_signs, uint16_t* qjl_norms) {
+  TqEncodeArgs e{};
+  e.key = kv;
+  e.rows = N;
+  e.bits = bits;
+  e.head_dim = head_dim;
+  e.padded_dim = padded_dim;
+  e.src_dtype = src_dtype;
+  e.packed = packed ? 1 : 0;
+  e.signs = signs;
+  e.jl = jl;
+  e.lut = angle_lut;
+  e.radius = radius;
+  e.angles = angles;
+  e.qjl_signs = qjl_signs;
+  e.qjl_norms = qjl_norms;
+  return e;
+}
+}  // namespace
+
+extern "C" int vrm_turboquant_compress(const void* kv, int src_dtype, int N, int head_dim, int padded_dim,
+                                       int n_levels, int bits, int qjl_dim, const float* signs, const float* jl,
+                                       const float* angle_lut, uint16_t* radius, uint8_t* angles,
+                                       uint8_t* qjl_signs, uint16_t* qjl_norms, vrm_stream_t stream) {
+  const char* who = "vrm_turboquant_compress";
+  const int rc = check_compress(kv, src_dtype, N, head_dim, padded_dim, n_levels, bits, qjl_dim, signs, jl, angle_lut,
+                                radius, angles, qjl_signs, qjl_norms, who);
+  if (rc) return rc;
+  if (N == 0) return VRM_OK;
+  if (N >= kTileMinRows && N <= kTileMaxRows && tq_tile_ok(padded_dim, bits, qjl_dim)) {
+    launch_tq_encode(codec_args(kv, src_dtype, N, head_dim, padded_dim, bits, false, signs, jl, angle_lut, radius,
+                                angles, qjl_signs, qjl_norms),
+                     reinterpret_cast<hipStream_t>(stream));
+    return launch_status(who);
   }
   TqArgs a{};
   a.kv = kv;
@@ -870,6 +762,31 @@ extern "C" int vrm_turboquant_compress(const void* kv, int src_dtype, int N, int
   }
 #undef VRM_TQ_PD
 #undef VRM_TQ_LAUNCH
+  return launch_status(who);
+}
+
+extern "C" int vrm_turboquant_compress_packed(const void* kv, int src_dtype, int N, int head_dim, int padded_dim,
+                                              int n_levels, int bits, int qjl_dim, const float* signs,
+                                              const float* jl, const float* angle_lut, uint16_t* radius,
+                                              uint8_t* angles_packed, uint8_t* signs_packed, uint16_t* qjl_norms,
+                                              vrm_stream_t stream) {
+  const char* who = "vrm_turboquant_compress_packed";
+  const int rc = check_compress(kv, src_dtype, N, head_dim, padded_dim, n_levels, bits, qjl_dim, signs, jl, angle_lut,
+                                radius, angles_packed, signs_packed, qjl_norms, who);
+  if (rc) return rc;
+  if (!tq_tile_ok(padded_dim, bits, qjl_dim) || N > kTileMaxRows) {
+    set_error("%s: packs padded_dim 64 or 128, 2 to 4 bits and padded_dim / 2 QJL rows (got %d, %d, %d; N=%d)", who,
+              padded_dim, bits, qjl_dim, N);
+    return VRM_ERR_UNSUPPORTED;
+  }
+  if (((reinterpret_cast<uintptr_t>(angles_packed) | reinterpret_cast<uintptr_t>(signs_packed)) & 3) != 0) {
+    set_error("%s: packed arrays must be aligned to 4 bytes", who);
+    return VRM_ERR_ARG;
+  }
+  if (N == 0) return VRM_OK;
+  launch_tq_encode(codec_args(kv, src_dtype, N, head_dim, padded_dim, bits, true, signs, jl, angle_lut, radius,
+                              angles_packed, signs_packed, qjl_norms),
+                   reinterpret_cast<hipStream_t>(stream));
   return launch_status(who);
 }
 
@@ -997,24 +914,37 @@ int tq_pool_write(const void* key, const void* value, int src_dtype, const int32
 #undef VRM_TQ_WRITE_GEN_PD
     return launch_status(who);
   }
-  // bulk writes pack kBulkRows rows (wavefronts) per workgroup, small ones one
-  const bool bulk = rows >= kBulkMinRows;
-  const dim3 grid(bulk ? (rows + kBulkRows - 1) / kBulkRows : rows, 2);
-#define VRM_TQ_WRITE_RP(SRC, B, PDV)                                                                         \
-  if (bulk)                                                                                                  \
-    hipLaunchKernelGGL((tq_pool_write_kernel<SRC, B, kBulkRows, PDV>), grid, dim3(64 * kBulkRows), 0, st, a); \
-  else                                                                                                       \
-    hipLaunchKernelGGL((tq_pool_write_kernel<SRC, B, 1, PDV>), grid, dim3(64), 0, st, a);
-#define VRM_TQ_WRITE_R(SRC, B)          \
-  if (pd == 64)                         \
-    VRM_TQ_WRITE_RP(SRC, B, 64)         \
-  else                                  \
-    VRM_TQ_WRITE_RP(SRC, B, 128)
+  if (pd == 64 || rows >= kTileMinRows) {
+    TqEncodeArgs e{};
+    e.key = key;
+    e.value = value;
+    e.page_ids = page_ids;
+    e.slots = slots;
+    e.n_valid = n_valid;
+    e.pool = tq_pool;
+    e.rows = rows;
+    e.KH = KH;
+    e.L = L;
+    e.P = P;
+    e.layer = layer_idx;
+    e.bits = bits;
+    e.head_dim = D;
+    e.padded_dim = pd;
+    e.src_dtype = src_dtype;
+    e.from_pool = a.from_pool;
+    e.signs = signs;
+    e.jl = jl;
+    e.lut = angle_lut;
+    launch_tq_encode(e, st);
+    return launch_status(who);
+  }
+#define VRM_TQ_WRITE_B(SRC, B) \
+  hipLaunchKernelGGL((tq_pool_write_kernel<SRC, B>), dim3(rows, 2), dim3(64), 0, st, a)
 #define VRM_TQ_WRITE(SRC)                          \
   switch (bits) {                                  \
-    case 2: VRM_TQ_WRITE_R(SRC, 2); break;         \
-    case 3: VRM_TQ_WRITE_R(SRC, 3); break;         \
-    default: VRM_TQ_WRITE_R(SRC, 4); break;        \
+    case 2: VRM_TQ_WRITE_B(SRC, 2); break;         \
+    case 3: VRM_TQ_WRITE_B(SRC, 3); break;         \
+    default: VRM_TQ_WRITE_B(SRC, 4); break;        \
   }
   switch (src_dtype) {
     case VRM_SRC_F32: VRM_TQ_WRITE(VRM_SRC_F32); break;
@@ -1022,8 +952,7 @@ int tq_pool_write(const void* key, const void* value, int src_dtype, const int32
     default: VRM_TQ_WRITE(VRM_SRC_BF16); break;
   }
 #undef VRM_TQ_WRITE
-#undef VRM_TQ_WRITE_R
-#undef VRM_TQ_WRITE_RP
+#undef VRM_TQ_WRITE_B
   return launch_status(who);
 }
 }  // namespace

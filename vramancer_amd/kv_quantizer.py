@@ -169,8 +169,15 @@ class KVCacheCompressor(nn.Module):
 
     def compress(self, kv, pack: bool = True):
         """Compresses [..., head_dim] vectors; returns the packed dict by default."""
-        result = CUDATurboQuantOps.compress_gpu(kv, *self._ops_args(), self._hadamard_signs, self.jl_matrix)
-        return self._pack_compressed(result) if pack else result
+        return self._compress(kv, pack)
+
+    def _compress(self, kv, pack):
+        args = (kv, *self._ops_args(), self._hadamard_signs, self.jl_matrix)
+        if not pack:
+            return CUDATurboQuantOps.compress_gpu(*args)
+        packed = CUDATurboQuantOps.compress_packed_gpu(*args)  # None: settings it does not serve
+        return self._pack_compressed(CUDATurboQuantOps.compress_gpu(*args)) if packed is None else packed
+
 
     def compress_batch(self, kv_list: list, pack: bool = False) -> list:
         """Compresses several tensors with one kernel launch and returns one
@@ -186,10 +193,7 @@ class KVCacheCompressor(nn.Module):
         shapes = [tuple(kv.shape) for kv in kv_list]
         flat = [kv.reshape(-1, self.head_dim) for kv in kv_list]
         rows = [f.shape[0] for f in flat]
-        result = CUDATurboQuantOps.compress_gpu(torch.cat(flat, dim=0), *self._ops_args(), self._hadamard_signs,
-                                                self.jl_matrix)
-        if pack:
-            result = self._pack_compressed(result)
+        result = self._compress(torch.cat(flat, dim=0), pack)
         return _split_rows(result, rows, shapes)
 
     def decompress(self, compressed):

@@ -107,6 +107,44 @@ class CUDATurboQuantOps:
     """Fused gfx950 TurboQuant ops: one kernel launch per compress / decompress."""
 
     @staticmethod
+    def _compress_inputs(kv, head_dim: int, padded_dim: int, hadamard_signs, jl_matrix):
+        import torch
+
+        _lib.require_cuda(kv)
+        flat = kv.reshape(-1, head_dim)
+        if flat.dtype not in (torch.float32, torch.float16, torch.bfloat16):
+            flat = flat.float()
+        flat = flat.contiguous()
+        device = flat.device
+        signs_f = hadamard_signs.to(device=device, dtype=torch.float32).contiguous()
+        jl_f = jl_matrix.to(device=device, dtype=torch.float32).contiguous()
+        if signs_f.shape != (padded_dim,) or jl_f.shape != (jl_f.shape[0], padded_dim):
+            raise RuntimeError("hadamard_signs / jl_matrix shapes do not match padded_dim")
+        return flat, signs_f, jl_f
+
+    @staticmethod
+    def _compress(entry: str, inputs, angle_bytes: int, sign_bytes: int, head_dim: int, padded_dim: int,
+                  n_levels: int, bits_per_angle: int):
+        """Runs a compress entry: (radius [N], angles [N, angle_bytes], signs
+        [N, sign_bytes], norms [N])."""
+        import torch
+
+        flat, signs_f, jl_f = inputs
+        device, N = flat.device, flat.shape[0]
+        radius = torch.empty(N, dtype=torch.float16, device=device)
+        angles = torch.empty((N, angle_bytes), dtype=torch.uint8, device=device)
+        qjl_signs = torch.empty((N, sign_bytes), dtype=torch.uint8, device=device)
+        qjl_norms = torch.empty(N, dtype=torch.float16, device=device)
+        lut = angle_lut(bits_per_angle, device)
+        rc = getattr(_lib.load(), entry)(
+            _lib.ptr(flat), _lib.src_dtype_code(flat.dtype), N, head_dim, padded_dim, n_levels, bits_per_angle,
+            jl_f.shape[0], _lib.ptr(signs_f), _lib.ptr(jl_f), _lib.ptr(lut), _lib.ptr(radius), _lib.ptr(angles),
+            _lib.ptr(qjl_signs), _lib.ptr(qjl_norms), _lib.stream_of(flat),
+        )
+        _lib.check(rc, "turboquant compress")
+        return radius, angles, qjl_signs, qjl_norms
+
+    @staticmethod
     def compress_gpu(
         kv,              # [N, head_dim] or [..., head_dim]; float32 / float16 / bfloat16
         head_dim: int,
@@ -116,38 +154,39 @@ class CUDATurboQuantOps:
         hadamard_signs,  # [padded_dim] +-1
         jl_matrix,       # [qjl_dim, padded_dim]
     ) -> dict:
-        import torch
-
-        _lib.require_cuda(kv)
-        orig_shape = kv.shape
-        flat = kv.reshape(-1, head_dim)
-        if flat.dtype not in (torch.float32, torch.float16, torch.bfloat16):
-            flat = flat.float()
-        flat = flat.contiguous()
-        device = flat.device
-        signs_f = hadamard_signs.to(device=device, dtype=torch.float32).contiguous()
-        jl_f = jl_matrix.to(device=device, dtype=torch.float32).contiguous()
-        qjl_dim = jl_f.shape[0]
-        if signs_f.shape != (padded_dim,) or jl_f.shape != (qjl_dim, padded_dim):
-            raise RuntimeError("hadamard_signs / jl_matrix shapes do not match padded_dim")
-        N = flat.shape[0]
-        radius = torch.empty(N, dtype=torch.float16, device=device)
-        angles = torch.empty((N, padded_dim - 1), dtype=torch.uint8, device=device)
-        qjl_signs = torch.empty((N, qjl_dim), dtype=torch.uint8, device=device)
-        qjl_norms = torch.empty(N, dtype=torch.float16, device=device)
-        lut = angle_lut(bits_per_angle, device)
-        rc = _lib.load().vrm_turboquant_compress(
-            _lib.ptr(flat), _lib.src_dtype_code(flat.dtype), N, head_dim, padded_dim, n_levels, bits_per_angle,
-            qjl_dim, _lib.ptr(signs_f), _lib.ptr(jl_f), _lib.ptr(lut), _lib.ptr(radius), _lib.ptr(angles),
-            _lib.ptr(qjl_signs), _lib.ptr(qjl_norms), _lib.stream_of(flat),
-        )
-        _lib.check(rc, "turboquant compress")
+        inputs = CUDATurboQuantOps._compress_inputs(kv, head_dim, padded_dim, hadamard_signs, jl_matrix)
+        radius, angles, qjl_signs, qjl_norms = CUDATurboQuantOps._compress(
+            "vrm_turboquant_compress", inputs, padded_dim - 1, inputs[2].shape[0], head_dim, padded_dim, n_levels,
+            bits_per_angle)
         return {
             "radius": radius,                          # [N] fp16
             "angles": _split_levels(angles, padded_dim, n_levels),
             "qjl_signs": qjl_signs,                    # [N, qjl_dim] uint8
             "qjl_norms": qjl_norms.unsqueeze(-1),      # [N, 1] fp16
-            "shape": orig_shape,
+            "shape": kv.shape,
+        }
+
+    @staticmethod
+    def compress_packed_gpu(kv, head_dim: int, padded_dim: int, n_levels: int, bits_per_angle: int, hadamard_signs,
+                            jl_matrix):
+        """The packed dict of ``kv`` in one launch, or None for settings the
+        packing encoder does not serve."""
+        if padded_dim not in (64, 128) or not 2 <= bits_per_angle <= 4 or jl_matrix.shape[0] != padded_dim // 2:
+            return None
+        inputs = CUDATurboQuantOps._compress_inputs(kv, head_dim, padded_dim, hadamard_signs, jl_matrix)
+        qjl_dim = inputs[2].shape[0]
+        radius, angles, signs, norms = CUDATurboQuantOps._compress(
+            "vrm_turboquant_compress_packed", inputs, ((padded_dim - 1) * bits_per_angle + 7) // 8, qjl_dim // 8,
+            head_dim, padded_dim, n_levels, bits_per_angle)
+        return {
+            "radius": radius,
+            "angles_packed": angles,
+            "qjl_signs_packed": signs,
+            "qjl_norms": norms.unsqueeze(-1),
+            "shape": kv.shape,
+            "_N": inputs[0].shape[0],
+            "_qjl_dim": qjl_dim,
+            "_level_dims": [padded_dim >> (l + 1) for l in range(n_levels)],
         }
 
     @staticmethod
