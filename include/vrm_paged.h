@@ -372,6 +372,14 @@ int vrm_turboquant_decompress(const uint16_t* radius, const uint8_t* angles, int
                               const float* signs, const float* angle_lut, float* out,
                               int rotated, vrm_stream_t stream);
 
+/* The same from the packed angles of vrm_turboquant_compress_packed, aligned to
+ * 4 bytes.  Serves padded_dim 64 or 128 and 2 to 4 bits; VRM_ERR_UNSUPPORTED
+ * otherwise (vrm_unpack_bits, then decompress). */
+int vrm_turboquant_decompress_packed(const uint16_t* radius, const uint8_t* angles_packed,
+                                     int N, int head_dim, int padded_dim, int n_levels,
+                                     int bits, const float* signs, const float* angle_lut,
+                                     float* out, int rotated, vrm_stream_t stream);
+
 /*
  * scores[M][N] float32 = out_scale * (q_rot . k_polar + QJL correction) for M
  * query rows q [M][head_dim] float32 against N compressed keys in the raw

@@ -1,4 +1,6 @@
-"""The TurboQuant tile encoder (16 rows per wavefront) on the GPU.
+"""The TurboQuant kernels with 16 rows per wavefront on the GPU.
+
+Encoder:
 
 Calls of 2048 rows and more take it; the same rows in smaller calls take one
 row per wavefront, the path the oracle tests hold to the reference.  Both give
@@ -12,6 +14,7 @@ import math
 import pytest
 import torch
 
+from oracle import turboquant as TQ
 from test_gpu_turboquant import _student_t
 from vramancer_amd import tq_pages
 from vramancer_amd.kv_quantizer import KVCacheCompressor, _pack_bits, _pack_values
@@ -100,3 +103,34 @@ def test_tile_pages_equal_small_writes(head_dim, bits):
     ref = comp.compress(torch.stack([k[4], v[4]]), pack=False)
     assert torch.equal(got["angles"].reshape(-1, got["angles"].shape[-1]).cpu(), torch.cat(ref["angles"], -1).cpu())
     assert torch.equal(got["qjl_signs"][0, 0].reshape(KH * 16, -1).cpu(), ref["qjl_signs"][:KH * 16].cpu())
+
+
+@pytest.mark.parametrize("head_dim,bits", [(128, 2), (128, 3), (128, 4), (96, 3), (70, 4), (64, 2), (64, 3), (64, 4),
+                                           (33, 3)])
+def test_tile_decompress_matches_oracle(head_dim, bits):
+    """Decompression of raw and packed codes is the oracle's, bit for bit (zeros
+    and NaN apart), over radii of every kind; 16,384 rows and more of raw codes
+    at padded dim 128 take the tiles, packed codes at any count."""
+    _say(f"tile decompress {head_dim} {bits}")
+    p = TQ.make_params(head_dim, bits, seed=head_dim)
+    torch.manual_seed(head_dim)
+    comp = KVCacheCompressor(head_dim, bits).to(DEV)
+    pd = comp._padded_dim
+    n = 16384 + 5
+    g = torch.Generator().manual_seed(bits)
+    radius = (torch.rand(n, generator=g) * 20).half()
+    radius[::97] = torch.tensor([0.0, -0.0, math.inf, math.nan, 6e-8, 65504.0, -3.0]).half().repeat(n)[:radius[::97].numel()]
+    bins = torch.randint(0, 1 << bits, (n, pd - 1), generator=g, dtype=torch.uint8)
+    dims = [pd >> (l + 1) for l in range(comp._n_levels)]
+    raw = {"radius": radius, "angles": list(torch.split(bins, dims, -1)), "qjl_signs": torch.zeros(n, pd // 2, dtype=torch.uint8),
+           "qjl_norms": torch.zeros(n, 1).half(), "shape": (n, head_dim)}
+    want = TQ.decompress(p, dict(raw, radius=radius[:, None])).reshape(n, head_dim)
+    dev = {k: (list(torch.split(bins.to(DEV), dims, -1)) if k == "angles" else v.to(DEV) if torch.is_tensor(v) else v)
+           for k, v in raw.items()}
+    for m in (1, 17, n):
+        part = {k: ([a[:m] for a in v] if k == "angles" else v[:m] if torch.is_tensor(v) else (m, head_dim))
+                for k, v in dev.items()}
+        for d in (part, comp._pack_compressed(part)):
+            got = comp.decompress(d).cpu()
+            assert got.shape == (m, head_dim)
+            torch.testing.assert_close(got, want[:m], atol=0, rtol=0, equal_nan=True)

@@ -23,6 +23,7 @@
 
 #ifndef VRM_HD
 #ifdef __HIPCC__
+#include <hip/hip_runtime.h>
 #define VRM_HD __host__ __device__ __forceinline__
 #else
 #define VRM_HD static inline

@@ -1,4 +1,5 @@
-// Launchers of the TurboQuant tile encoder (vrm_tq_encode.hip).
+// Launchers of the TurboQuant kernels with 16 rows per wavefront: the encoder
+// (vrm_tq_encode.hip) and decompression (vrm_tq_decompress.hip).
 #pragma once
 #include "vrm_common.h"
 
@@ -29,13 +30,29 @@ struct TqEncodeArgs {
   uint16_t* qjl_norms;
 };
 
-// True for the settings the tile encoder serves: padded dim 64 or 128, 2 to 4
-// bits per angle, padded_dim / 2 QJL rows.
+// Rows to decompress: angles [N][PD - 1] bytes, or packed (MSB first, 4-byte
+// aligned); out [N][head_dim], or the rotated rows [N][PD].
+struct TqDecompressArgs {
+  const uint16_t* radius;
+  const uint8_t* angles;
+  int N, head_dim, padded_dim, bits;
+  int packed, rotated;
+  const float* signs;
+  const float* lut;
+  float* out;
+};
+
+// True for the settings these kernels serve: padded dim 64 or 128, 2 to 4
+// bits per angle; the encoder also wants padded_dim / 2 QJL rows.
+inline bool tq_rows_ok(int padded_dim, int bits) {
+  return (padded_dim == 64 || padded_dim == 128) && bits >= 2 && bits <= 4;
+}
 inline bool tq_tile_ok(int padded_dim, int bits, int qjl_dim) {
-  return (padded_dim == 64 || padded_dim == 128) && qjl_dim == padded_dim / 2 && bits >= 2 && bits <= 4;
+  return tq_rows_ok(padded_dim, bits) && qjl_dim == padded_dim / 2;
 }
 
-// Launches the encoder; the caller checks launch_status.
+// The caller checks launch_status.
 void launch_tq_encode(const TqEncodeArgs& a, hipStream_t stream);
+void launch_tq_decompress(const TqDecompressArgs& a, hipStream_t stream);
 
 }  // namespace vrm

@@ -30,8 +30,8 @@
 #include "vrm_tq_encode.h"
 
 #include "vrm_tq_bin.h"
-#include "vrm_tq_layout.h"
 #include "vrm_tq_row.h"
+#include "vrm_tq_tile.h"
 
 namespace vrm {
 namespace {
@@ -42,8 +42,6 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-
-constexpr int kTile = 16;  // rows per wavefront
 
 // Correctly rounded square root of x >= 1e-12: the radii carry that floor.
 __device__ __forceinline__ float sqrt_radius(float x) {
@@ -56,63 +54,10 @@ __device__ __forceinline__ float radius_of(float x0, float x1) {
   return sqrt_radius(__fadd_rn(__fadd_rn(__fmul_rn(x0, x0), __fmul_rn(x1, x1)), 1e-12f));
 }
 
-// Value of the lane 16 (32) lanes away: neighbour quarters, then halves.
-__device__ __forceinline__ float other16(float v) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float((__lane_id() & 16) ? r[0] : r[1]);
-}
-__device__ __forceinline__ float other32(float v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float((__lane_id() & 32) ? r[0] : r[1]);
-}
-
-// One butterfly stage across lanes for two elements a, b: the lower lane
-// keeps lower + upper, the upper lane lower - upper.  The swap gathers both
-// lanes' operands of a in the lower lane and of b in the upper one.
-template <int H>
-__device__ __forceinline__ void cross_butterfly(float& a, float& b) {
-  const auto r = H == 16 ? __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false)
-                         : __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-  const float lo = __uint_as_float(r[0]), hi = __uint_as_float(r[1]);
-  const uint32_t s = __float_as_uint(__fadd_rn(lo, hi)), d = __float_as_uint(__fsub_rn(lo, hi));
-  const auto t = H == 16 ? __builtin_amdgcn_permlane16_swap(s, d, false, false)
-                         : __builtin_amdgcn_permlane32_swap(s, d, false, false);
-  a = __uint_as_float(t[0]);
-  b = __uint_as_float(t[1]);
-}
-
 __device__ __forceinline__ float load_any(int src, const void* p, size_t i) {
   return src == VRM_SRC_F32 ? load_row<VRM_SRC_F32>(p, i)
                             : src == VRM_SRC_F16 ? load_row<VRM_SRC_F16>(p, i) : load_row<VRM_SRC_BF16>(p, i);
 }
-
-// Slot of angle a of level l of a quarter.
-template <int PD, int BITS>
-__device__ __forceinline__ int slot_in_quarter(int l, int a) {
-  int q, s;
-  tq::slot_of(PD, l, a, BITS, q, s);
-  return s;
-}
-
-template <int PD, int BITS>
-struct Quarter {
-  static constexpr int NQ = PD / 4;                          // dims, and slots, of a lane
-  static constexpr int LQ = PD == 128 ? 4 : 3;               // its top level
-  static constexpr int WORDS = (NQ * BITS + 31) / 32;        // dwords of its record
-  uint32_t w[WORDS];
-
-  __device__ __forceinline__ void put(int slot, uint32_t bin) {
-    const int pos = slot * BITS;
-    w[pos / 32] |= bin << (pos % 32);
-    if (pos % 32 + BITS > 32) w[pos / 32 + 1] |= bin >> (32 - pos % 32);
-  }
-  __device__ __forceinline__ uint32_t get(int slot) const {
-    const int pos = slot * BITS;
-    uint32_t x = w[pos / 32] >> (pos % 32);
-    if (pos % 32 + BITS > 32) x |= w[pos / 32 + 1] << (32 - pos % 32);
-    return x & ((1u << BITS) - 1);
-  }
-};
 
 // LDS of a workgroup: the JL matrix as bf16 hi and lo fragments, its longest
 // row's 2-norm, the angle table, and a scratch row per wavefront.
@@ -286,21 +231,7 @@ __global__ void __launch_bounds__(512) tq_encode_tile_kernel(TqEncodeArgs a, int
         for (int i = 0; i < NQ; ++i) v[i] = __fmul_rn(v[i], a.signs[e0 + i]);
       }
     }
-#pragma unroll
-    for (int h = 1; h < NQ; h <<= 1) {
-#pragma unroll
-      for (int i = 0; i < NQ; ++i) {
-        if (!(i & h)) {
-          const float lo = v[i], hi = v[i + h];
-          v[i] = __fadd_rn(lo, hi);
-          v[i + h] = __fsub_rn(lo, hi);
-        }
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < NQ; i += 2) cross_butterfly<16>(v[i], v[i + 1]);
-#pragma unroll
-    for (int i = 0; i < NQ; i += 2) cross_butterfly<32>(v[i], v[i + 1]);
+    tile_fwht<PD>(v);
 #pragma unroll
     for (int i = 0; i < NQ; ++i) v[i] = PD == 64 ? __fmul_rn(v[i], 0.125f) : vrm_tq_bin::div_sqrt128(v[i]);
 

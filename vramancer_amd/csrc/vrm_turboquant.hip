@@ -61,6 +61,11 @@ constexpr int kBulkMinRows = 4096;
 // size (2 x 8 rows 7.1 / 6.4 us, 2 x 4096 16.7 / 8.1).
 constexpr int kTileMinRows = 2048;
 constexpr int kTileMaxRows = 0x7fffff00;
+// Rows from which raw codes at padded dim 128 are decompressed 16 rows per
+// wavefront (row kernel / tiles at 3 bits: 4096 rows 4.3 / 5.3 us, 16,384 7.5 /
+// 6.1, 65,536 23.4 / 16.4; padded dim 64 is as fast or faster tiled from one
+// row on, 65,536 rows 14.1 / 7.2).
+constexpr int kTileMinDecompressRows = 16384;
 
 // LUT_LDS: the angle table (4 x 2^bits floats, bits <= 4) is read from LDS.
 template <int SRC, int PD, int ROWS, bool LUT_LDS>
@@ -790,6 +795,26 @@ extern "C" int vrm_turboquant_compress_packed(const void* kv, int src_dtype, int
   return launch_status(who);
 }
 
+namespace {
+TqDecompressArgs rows_args(const uint16_t* radius, const uint8_t* angles, int N, int head_dim, int padded_dim,
+                           int bits, bool packed, int rotated, const float* signs, const float* angle_lut,
+                           float* out) {
+  TqDecompressArgs d{};
+  d.radius = radius;
+  d.angles = angles;
+  d.N = N;
+  d.head_dim = head_dim;
+  d.padded_dim = padded_dim;
+  d.bits = bits;
+  d.packed = packed ? 1 : 0;
+  d.rotated = rotated;
+  d.signs = signs;
+  d.lut = angle_lut;
+  d.out = out;
+  return d;
+}
+}  // namespace
+
 extern "C" int vrm_turboquant_decompress(const uint16_t* radius, const uint8_t* angles, int N, int head_dim,
                                          int padded_dim, int n_levels, int bits, const float* signs,
                                          const float* angle_lut, float* out, int rotated, vrm_stream_t stream) {
@@ -800,6 +825,12 @@ extern "C" int vrm_turboquant_decompress(const uint16_t* radius, const uint8_t* 
   if (!radius || !angles || !signs || !angle_lut || !out) {
     set_error("%s: null pointer argument", who);
     return VRM_ERR_ARG;
+  }
+  if (tq_rows_ok(padded_dim, bits) && (padded_dim == 64 || N >= kTileMinDecompressRows)) {
+    launch_tq_decompress(rows_args(radius, angles, N, head_dim, padded_dim, bits, false, rotated, signs, angle_lut,
+                                   out),
+                         reinterpret_cast<hipStream_t>(stream));
+    return launch_status(who);
   }
   TqArgs a{};
   a.N = N;
@@ -829,6 +860,32 @@ extern "C" int vrm_turboquant_decompress(const uint16_t* radius, const uint8_t* 
     default: VRM_TQ_DECOMP(256); break;
   }
 #undef VRM_TQ_DECOMP
+  return launch_status(who);
+}
+
+extern "C" int vrm_turboquant_decompress_packed(const uint16_t* radius, const uint8_t* angles_packed, int N,
+                                                int head_dim, int padded_dim, int n_levels, int bits,
+                                                const float* signs, const float* angle_lut, float* out, int rotated,
+                                                vrm_stream_t stream) {
+  const char* who = "vrm_turboquant_decompress_packed";
+  int rc = check_tq(N, head_dim, padded_dim, n_levels, bits, who);
+  if (rc) return rc;
+  if (!tq_rows_ok(padded_dim, bits)) {
+    set_error("%s: reads padded_dim 64 or 128 and 2 to 4 bits (got %d, %d)", who, padded_dim, bits);
+    return VRM_ERR_UNSUPPORTED;
+  }
+  if (N == 0) return VRM_OK;
+  if (!radius || !angles_packed || !signs || !angle_lut || !out) {
+    set_error("%s: null pointer argument", who);
+    return VRM_ERR_ARG;
+  }
+  if (reinterpret_cast<uintptr_t>(angles_packed) & 3) {
+    set_error("%s: angles_packed must be aligned to 4 bytes", who);
+    return VRM_ERR_ARG;
+  }
+  launch_tq_decompress(rows_args(radius, angles_packed, N, head_dim, padded_dim, bits, true, rotated, signs,
+                                 angle_lut, out),
+                       reinterpret_cast<hipStream_t>(stream));
   return launch_status(who);
 }
 

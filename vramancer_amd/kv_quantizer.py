@@ -198,7 +198,11 @@ class KVCacheCompressor(nn.Module):
 
     def decompress(self, compressed):
         """Approximate K/V from polar codes only (no QJL), shaped like the input."""
-        compressed = self._unpack_compressed(compressed)
+        if "angles" not in compressed:
+            out = CUDATurboQuantOps.decompress_packed_gpu(compressed, *self._ops_args(), self._hadamard_signs)
+            if out is not None:
+                return out
+            compressed = self._unpack_compressed(compressed)
         return CUDATurboQuantOps.decompress_gpu(compressed, *self._ops_args(), self._hadamard_signs)
 
     def attention_score(self, q, compressed_k):

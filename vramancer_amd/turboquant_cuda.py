@@ -192,25 +192,51 @@ class CUDATurboQuantOps:
     @staticmethod
     def _decode(compressed: dict, head_dim: int, padded_dim: int, n_levels: int, bits_per_angle: int,
                 hadamard_signs, rotated: bool):
+        radius = compressed["radius"].reshape(-1).half().contiguous()
+        _lib.require_cuda(radius)
+        angles = level_bins(compressed["angles"], padded_dim - 1)
+        if angles.shape != (radius.shape[0], padded_dim - 1):
+            raise RuntimeError(f"angles {tuple(angles.shape)} do not match padded_dim {padded_dim}")
+        return CUDATurboQuantOps._decode_rows("vrm_turboquant_decompress", radius, angles, head_dim, padded_dim,
+                                              n_levels, bits_per_angle, hadamard_signs, rotated)
+
+    @staticmethod
+    def _decode_rows(entry: str, radius, angles, head_dim: int, padded_dim: int, n_levels: int, bits_per_angle: int,
+                     hadamard_signs, rotated: bool):
         import torch
 
-        radius = compressed["radius"].reshape(-1).to(torch.float16).contiguous()
-        _lib.require_cuda(radius)
-        device = radius.device
-        angles = level_bins(compressed["angles"], padded_dim - 1)
-        N = radius.shape[0]
-        if angles.shape != (N, padded_dim - 1):
-            raise RuntimeError(f"angles {tuple(angles.shape)} do not match padded_dim {padded_dim}")
+        device, N = radius.device, radius.shape[0]
         signs_f = hadamard_signs.to(device=device, dtype=torch.float32).contiguous()
         width = padded_dim if rotated else head_dim
         out = torch.empty((N, width), dtype=torch.float32, device=device)
         lut = angle_lut(bits_per_angle, device)
-        rc = _lib.load().vrm_turboquant_decompress(
+        rc = getattr(_lib.load(), entry)(
             _lib.ptr(radius), _lib.ptr(angles), N, head_dim, padded_dim, n_levels, bits_per_angle,
             _lib.ptr(signs_f), _lib.ptr(lut), _lib.ptr(out), 1 if rotated else 0, _lib.stream_of(radius),
         )
         _lib.check(rc, "turboquant decompress")
         return out
+
+    @staticmethod
+    def decompress_packed_gpu(packed: dict, head_dim: int, padded_dim: int, n_levels: int, bits_per_angle: int,
+                              hadamard_signs):
+        """Decompresses a packed dict as ``compress_packed_gpu`` returns it in
+        one launch; None for any other (unpack it, then ``decompress_gpu``)."""
+        import torch
+
+        radius, angles, signs = packed["radius"], packed["angles_packed"], packed["qjl_signs_packed"]
+        N, nbytes = packed["_N"], ((padded_dim - 1) * bits_per_angle + 7) // 8
+        if (padded_dim not in (64, 128) or not 2 <= bits_per_angle <= 4 or "qjl_norms" not in packed or not radius.is_cuda
+                or radius.dtype != torch.float16 or radius.shape != (N,) or not radius.is_contiguous()
+                or any(t.dtype != torch.uint8 or t.device != radius.device or t.dim() != 2 or t.shape[0] != N
+                       for t in (angles, signs))
+                or angles.shape[1] != nbytes or not angles.is_contiguous() or angles.data_ptr() % 4
+                or signs.shape[1] * 8 < packed["_qjl_dim"]
+                or packed["_level_dims"] != [padded_dim >> (l + 1) for l in range(n_levels)]):
+            return None
+        out = CUDATurboQuantOps._decode_rows("vrm_turboquant_decompress_packed", radius, angles, head_dim,
+                                             padded_dim, n_levels, bits_per_angle, hadamard_signs, False)
+        return out.reshape(packed["shape"])
 
     @staticmethod
     def decompress_gpu(
