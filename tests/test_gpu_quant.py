@@ -189,3 +189,65 @@ def test_quant_other_head_dims_and_page_sizes(codec, D, PS):
         else:
             ref = KC.dequantize_fp8(pc[pid, 1].view(torch.uint8), sc_c[pid, 1][..., None, None])
         assert torch.equal(out[i], ref)
+
+
+@pytest.mark.parametrize("src_dtype", [torch.bfloat16, torch.float16, torch.float32],
+                         ids=lambda d: str(d).split(".")[-1])
+@pytest.mark.parametrize("codec", ["int8", "fp8"])
+@pytest.mark.parametrize("D,PS", [(128, 16), (64, 16), (96, 16), (16, 4), (112, 12), (80, 32), (128, 36), (144, 16)])
+def test_page_rows_any_values_and_alignment(codec, D, PS, src_dtype):
+    """Page writes from 16-byte aligned rows (four tokens per wavefront, where
+    D and PS allow) and from rows off that alignment give the same pool bytes,
+    for NaN, infinities, negative zeros, quotients at rounding ties, tiny and
+    huge rows, and partly filled pages."""
+    _say(f"page rows {codec} D{D} PS{PS} {src_dtype}")
+    P, L, KH, NP = 12, 2, 3, 8
+    g = torch.Generator().manual_seed(D + PS)
+    src = torch.randn(2, NP, KH, PS, D, generator=g) * torch.exp(torch.randn(2, NP, KH, PS, 1, generator=g))
+    src[:, 0, 0, 0] = 0.0
+    src[:, 0, 0, 1] = -0.0
+    src[:, 0, 1, 0, 3] = float("nan")
+    src[:, 1, 0, 1, 5] = float("inf")
+    src[:, 1, 1, 2, 7] = -float("inf")
+    # scale 1 (int8) and ties k + 1/2 of it; the fp8 codes' ties are among them
+    src[:, 2, 0, 3] = torch.randint(-126, 126, (2, D), generator=g) + 0.5
+    src[:, 2, 0, 3, 0] = 127.0
+    src[:, 3] *= 1e-30
+    src[:, 4, 1] *= 1e-38
+    src[:, 5, 2, :, ::2] = -0.0
+    src[:, 6, 0, 0] *= 1e4
+    src = src.to(src_dtype).to(DEV)
+    shifted = torch.empty(src.numel() + 1, dtype=src_dtype, device=DEV)[1:].reshape(src.shape).copy_(src)
+    ids = torch.randperm(P, generator=g)[:NP].to(torch.int32)
+    ids[7] = P  # outside the pool: dropped
+    n_valid = torch.tensor([PS, PS - 1, PS, PS, 1, PS, PS - 2, PS], dtype=torch.int32)
+    n_valid[3] = 0
+    pools = []
+    for rows in (src, shifted):
+        pool, scales = kv_quant.allocate_pool(P, L, KH, D, codec, PS, device=DEV)
+        pool.view(torch.uint8).fill_(9)
+        kv_quant.quantize_pages(pool, scales, 1, ids.to(DEV), rows[0], rows[1], n_valid.to(DEV))
+        pools.append((pool.view(torch.uint8).cpu(), scales.cpu()))
+    assert torch.equal(pools[0][0], pools[1][0])
+    assert torch.equal(pools[0][1].view(torch.int32), pools[1][1].view(torch.int32))
+
+
+@pytest.mark.parametrize("src_dtype", [torch.bfloat16, torch.float32], ids=lambda d: str(d).split(".")[-1])
+@pytest.mark.parametrize("codec,D,PS", [("int8", 128, 16), ("int8", 96, 12), ("int8", 64, 36), ("fp8", 128, 16),
+                                        ("fp8", 80, 8)])
+def test_many_pages_equal_few(codec, D, PS, src_dtype):
+    """8,192 (page, K/V, head) slices and more take one wavefront each; the
+    same pages in smaller calls take four."""
+    _say(f"many pages {codec} D{D} PS{PS} {src_dtype}")
+    KH, NP = 16, 259
+    g = torch.Generator(device=DEV).manual_seed(D)
+    k, v = (torch.randn(NP, KH, PS, D, generator=g, device=DEV).to(src_dtype) for _ in range(2))
+    ids = torch.randperm(NP, generator=torch.Generator().manual_seed(1)).to(torch.int32).to(DEV)
+    n_valid = torch.randint(0, PS + 1, (NP,), generator=torch.Generator().manual_seed(2)).to(torch.int32).to(DEV)
+    out = []
+    for step in (NP, 37):
+        pool, scales = kv_quant.allocate_pool(NP, 1, KH, D, codec, PS, device=DEV)
+        for s in range(0, NP, step):
+            kv_quant.quantize_pages(pool, scales, 0, ids[s:s + step], k[s:s + step], v[s:s + step], n_valid[s:s + step])
+        out.append((pool.view(torch.uint8).cpu(), scales.cpu()))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])

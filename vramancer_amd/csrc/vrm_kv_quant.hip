@@ -113,6 +113,272 @@ __global__ void __launch_bounds__(64) quant_i8_kernel(QuantArgs a) {
   if (lane == 0) scales_of(a, pid, kv, h)[slot] = scale;
 }
 
+// ---------------------------------------------------------------------------
+// Whole pages at D <= 128 from 16-byte aligned rows: one 256-thread workgroup
+// per (page, K/V, head), a wavefront per group of four tokens in turn, lane
+// (c, g) = lane % 16, lane / 16 with dims 8 c .. 8 c + 7 of token g of the
+// group.  Sixteen lanes then cover a token's row in two (32-bit sources: four)
+// 16-byte loads each, and the four tokens whose codes share a dword of the V
+// tiling sit 16 lanes apart, where v_permlane swaps exchange them in
+// registers.
+// Bound: memory, once past the launch (about 5 us).  Against one row per
+// wavefront with byte loads and stores: 512 pages of 8 heads x 16 x 128 from
+// bf16 (51 MB) int8 40.9 -> 14.2 us, fp8 42.4 -> 13.4; 4096 pages int8 371 ->
+// 87 us (4.6 TB/s), fp8 350 -> 82.
+// ---------------------------------------------------------------------------
+
+// x / s correctly rounded, from y = 1 / s correctly rounded: two residual
+// corrections, the first of which brings the quotient within one ulp, where
+// the second is exact (Markstein 1990).  Holds while the residuals stay
+// normal: fast_scale below; for a smaller quotient (|x| < 2^-10 s at its
+// smallest scale) both forms round to code 0 all the same.
+__device__ __forceinline__ float div_by(float x, float s, float y) {
+  float q = __fmul_rn(x, y);
+  q = fmaf(fmaf(-q, s, x), y, q);
+  return fmaf(fmaf(-q, s, x), y, q);
+}
+__device__ __forceinline__ bool fast_scale(float s) { return s > 0x1p-80f && s < 0x1p100f; }
+
+// Four int8 codes, little end first: |q| <= 127 after the clamp, so adding
+// 1.5 * 2^23 leaves the integer nearest to q (ties to even) in the low byte.
+__device__ __forceinline__ uint32_t int8_codes4(const float* x, float s, float y) {
+  uint32_t c[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float q = fminf(fmaxf(div_by(x[i], s, y), -127.f), 127.f);
+    c[i] = __float_as_uint(__fadd_rn(q, 12582912.f));
+  }
+  const uint32_t lo = __builtin_amdgcn_perm(c[1], c[0], 0x0c0c0400u);
+  const uint32_t hi = __builtin_amdgcn_perm(c[3], c[2], 0x04000c0cu);
+  return lo | hi;
+}
+
+__device__ __forceinline__ uint32_t pack4(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+  return a | (b << 8) | (c << 16) | (d << 24);
+}
+
+// Codes of 8 elements, little end first.  v_cvt_pk_fp8_f32 gives
+// vrm_e4m3::encode's code for every float up to 464 in magnitude (all of them
+// compared) but not for NaN, whose codes are the only ones with seven low bits
+// set: those lanes take the general path.
+template <bool FP8>
+__device__ __forceinline__ void codes8(const float (&x)[8], float scale, uint32_t& lo, uint32_t& hi) {
+  bool slow = !fast_scale(scale);
+  if (!slow) {
+    const float y = __fdiv_rn(1.f, scale);
+    if constexpr (FP8) {
+      float q[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) q[i] = copysignf(div_by(x[i], scale, y), x[i]);  // -0 stays -0
+      int a = __builtin_amdgcn_cvt_pk_fp8_f32(q[0], q[1], 0, false);
+      a = __builtin_amdgcn_cvt_pk_fp8_f32(q[2], q[3], a, true);
+      int b = __builtin_amdgcn_cvt_pk_fp8_f32(q[4], q[5], 0, false);
+      b = __builtin_amdgcn_cvt_pk_fp8_f32(q[6], q[7], b, true);
+      lo = (uint32_t)a;
+      hi = (uint32_t)b;
+      slow = ((((~lo & 0x7f7f7f7fu) - 0x01010101u) | ((~hi & 0x7f7f7f7fu) - 0x01010101u)) & 0x80808080u) != 0;
+    } else {
+      lo = int8_codes4(x, scale, y);
+      hi = int8_codes4(x + 4, scale, y);
+    }
+  }
+  if (slow) {
+    uint32_t c[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) c[i] = FP8 ? fp8_code(x[i], scale) : (uint8_t)int8_code(x[i], scale);
+    lo = pack4(c[0], c[1], c[2], c[3]);
+    hi = pack4(c[4], c[5], c[6], c[7]);
+  }
+}
+
+// First dims of a lane's two runs of four: 16-bit sources 8 c and 8 c + 4 (one
+// 16-byte load), 32-bit ones 4 c and D / 2 + 4 c (two loads, each contiguous
+// over the 16 lanes: 20 us against 33 us with adjacent ones at 512 pages).
+template <int SRC>
+__device__ __forceinline__ int run_dim(int c, int half, int D) {
+  return SRC == VRM_SRC_F32 ? 4 * c + half * (D >> 1) : 8 * c + 4 * half;
+}
+
+template <int SRC>
+__device__ __forceinline__ void load8(const void* p, size_t row, int c, int D, bool on, float (&x)[8]) {
+  if constexpr (SRC == VRM_SRC_F32) {
+    const float* q = static_cast<const float*>(p) + row;
+    const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
+    const float4 a = on ? *reinterpret_cast<const float4*>(q + run_dim<SRC>(c, 0, D)) : z;
+    const float4 b = on ? *reinterpret_cast<const float4*>(q + run_dim<SRC>(c, 1, D)) : z;
+    x[0] = a.x, x[1] = a.y, x[2] = a.z, x[3] = a.w;
+    x[4] = b.x, x[5] = b.y, x[6] = b.z, x[7] = b.w;
+  } else {
+    const uint4 z = make_uint4(0, 0, 0, 0);
+    const uint4 d = on ? *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(p) + row + 8 * c) : z;
+    const uint32_t w[4] = {d.x, d.y, d.z, d.w};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const uint32_t h = (w[k / 2] >> (16 * (k & 1))) & 0xffffu;
+      x[k] = SRC == VRM_SRC_F16 ? f16_bits_to_f32(h) : bf16_bits_to_f32(h);
+    }
+  }
+}
+
+// Stores the codes (lo: the first run, hi: the second) of token 4 tg + g of a
+// K slice, token-major.
+template <int SRC>
+__device__ __forceinline__ void store_k(uint8_t* dst, int tg, int c, int g, int D, bool on, uint32_t lo, uint32_t hi) {
+  if (!on) return;
+  uint8_t* row = dst + (size_t)(4 * tg + g) * D;
+  if constexpr (SRC == VRM_SRC_F32) {
+    *reinterpret_cast<uint32_t*>(row + run_dim<SRC>(c, 0, D)) = lo;
+    *reinterpret_cast<uint32_t*>(row + run_dim<SRC>(c, 1, D)) = hi;
+  } else {
+    *reinterpret_cast<uint2*>(row + 8 * c) = make_uint2(lo, hi);
+  }
+}
+
+// The same for a V slice, whose tiling puts four tokens of a dim in a dword:
+// 4 x 4 byte transposes over the group's tokens.  After the first swap a lane
+// holds one run of tokens 2 (g / 2) and 2 (g / 2) + 1, after the second two
+// dims of all four.
+template <int SRC>
+__device__ __forceinline__ void store_v(uint32_t* tile, int tg, int c, int g, int D, bool on, uint32_t lo, uint32_t hi) {
+  const auto s = __builtin_amdgcn_permlane16_swap(lo, hi, false, false);
+  const uint32_t p = __builtin_amdgcn_perm(s[1], s[0], 0x05010400u);  // the run's dims 0, 1 of both tokens
+  const uint32_t q = __builtin_amdgcn_perm(s[1], s[0], 0x07030602u);  // dims 2, 3
+  const auto u = __builtin_amdgcn_permlane32_swap(p, q, false, false);
+  if (on) {
+    const int d = run_dim<SRC>(c, g & 1, D) + (g & 2);
+    uint32_t* out = tile + (tg * 16 + (d & 15)) * (D >> 4) + (d >> 4);
+    out[0] = __builtin_amdgcn_perm(u[1], u[0], 0x05040100u);
+    out[D >> 4] = __builtin_amdgcn_perm(u[1], u[0], 0x07060302u);
+  }
+}
+
+// Largest of the 16 lanes of a row (rotations within the row: every lane gets
+// it).
+__device__ __forceinline__ float row16_max(float v) {
+  v = fmaxf(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x128, 0xf, 0xf, false)));
+  v = fmaxf(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x124, 0xf, 0xf, false)));
+  v = fmaxf(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x122, 0xf, 0xf, false)));
+  v = fmaxf(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x121, 0xf, 0xf, false)));
+  return v;
+}
+
+// A slice (page, K/V, head) goes to 4 / GROUPS wavefronts, GROUPS groups of
+// four tokens in flight each.  With one wavefront per slice (GROUPS 4) V tiles
+// leave through LDS in 1 KiB stores, and an fp8 page of up to 16 tokens needs
+// no barrier for its maximum.
+template <int SRC, int GROUPS, bool FP8>
+__global__ void __launch_bounds__(256) quant_slices_kernel(QuantArgs a) {
+  static_assert(!FP8 || GROUPS == 4, "an fp8 page's maximum is one wavefront's");
+  constexpr int PER = 4 / GROUPS;  // wavefronts per slice
+  __shared__ __align__(16) uint32_t v_lds[GROUPS > 1 ? 4 : 1][GROUPS > 1 ? GROUPS * 128 : 1];
+  const int D = a.D, PS = a.PS;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c = lane & 15, g = lane >> 4;
+  const int s = blockIdx.x * GROUPS + wave / PER;
+  if (s >= 2 * a.KH) return;
+  const int kv = s / a.KH, h = s % a.KH;
+  const int n = blockIdx.y;
+  const int pid = a.page_ids[n];
+  if (pid < 0 || pid >= a.P) return;
+  const int n_valid = a.slots[n];
+  const void* src = kv ? a.value : a.key;
+  const size_t base = ((size_t)n * a.KH + h) * PS * D;
+  uint8_t* dst = slice_of(a, pid, kv, h);
+  float* sc = scales_of(a, pid, kv, h);
+  const bool on = 8 * c < D;
+  for (int tg0 = wave % PER * GROUPS; tg0 < PS / 4; tg0 += 4) {
+    float x[GROUPS][8];
+#pragma unroll
+    for (int r = 0; r < GROUPS; ++r) {
+      const int t = 4 * (tg0 + r) + g;
+      load8<SRC>(src, base + (size_t)t * D, c, D, on && t < min(n_valid, PS), x[r]);
+    }
+    float page_scale = 0.f;
+    if constexpr (FP8) {
+      float amax = 0.f;
+#pragma unroll
+      for (int r = 0; r < GROUPS; ++r)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(x[r][i]));
+      page_scale = __fdiv_rn(group_max<64>(amax), 448.f);
+      if (lane == 0) sc[0] = page_scale;
+    }
+#pragma unroll
+    for (int r = 0; r < GROUPS; ++r) {
+      if (GROUPS > 1 && tg0 + r >= PS / 4) break;
+      float scale = page_scale;
+      if constexpr (!FP8) {
+        float amax = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(x[r][i]));
+        scale = __fdiv_rn(row16_max(amax), 127.f);
+      }
+      uint32_t lo = 0, hi = 0;
+      if (scale > 0.f && (!FP8 || 4 * (tg0 + r) + g < n_valid)) codes8<FP8>(x[r], scale, lo, hi);
+      if (kv == 0)
+        store_k<SRC>(dst, tg0 + r, c, g, D, on, lo, hi);
+      else if (GROUPS > 1)
+        store_v<SRC>(v_lds[wave], r, c, g, D, on, lo, hi);
+      else
+        store_v<SRC>(reinterpret_cast<uint32_t*>(dst), tg0 + r, c, g, D, on, lo, hi);
+      if (!FP8 && c == 0) sc[4 * (tg0 + r) + g] = scale;
+    }
+    if (GROUPS > 1 && kv == 1) {  // the groups' V tiles are one run of 4 D bytes each
+      __syncwarp();
+      uint4* out = reinterpret_cast<uint4*>(dst + (size_t)4 * tg0 * D);
+      const int n16 = min(GROUPS, PS / 4 - tg0) * D / 4;
+      for (int i = lane; i < n16; i += 64) out[i] = reinterpret_cast<const uint4*>(v_lds[wave])[i];
+      __syncwarp();
+    }
+  }
+}
+
+// fp8: the page maximum first, its rows held in registers between (PS <= 16
+// ROUNDS tokens).
+template <int SRC, int ROUNDS>
+__global__ void __launch_bounds__(256) quant_fp8_rows_kernel(QuantArgs a) {
+  __shared__ float red[4];
+  const int D = a.D, PS = a.PS;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c = lane & 15, g = lane >> 4;
+  const int kv = blockIdx.x / a.KH, h = blockIdx.x % a.KH;
+  const int n = blockIdx.y;
+  const int pid = a.page_ids[n];
+  if (pid < 0 || pid >= a.P) return;
+  const int n_valid = min(max(a.slots[n], 0), PS);
+  const void* src = kv ? a.value : a.key;
+  const size_t base = ((size_t)n * a.KH + h) * PS * D;
+  const bool on = 8 * c < D;
+  float x[ROUNDS][8];
+  float amax = 0.f;
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r) {
+    const int t = 4 * (wave + 4 * r) + g;
+    load8<SRC>(src, base + (size_t)t * D, c, D, on && t < n_valid, x[r]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(x[r][i]));
+  }
+  amax = group_max<64>(amax);
+  if (lane == 0) red[wave] = amax;
+  __syncthreads();
+  amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  const float scale = __fdiv_rn(amax, 448.f);
+  uint8_t* dst = slice_of(a, pid, kv, h);
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r) {
+    const int tg = wave + 4 * r;
+    if (tg < PS / 4) {
+      uint32_t lo = 0, hi = 0;
+      if (scale > 0.f && 4 * tg + g < n_valid) codes8<true>(x[r], scale, lo, hi);
+      if (kv == 0)
+        store_k<SRC>(dst, tg, c, g, D, on, lo, hi);
+      else
+        store_v<SRC>(reinterpret_cast<uint32_t*>(dst), tg, c, g, D, on, lo, hi);
+    }
+  }
+  if (threadIdx.x == 0) *scales_of(a, pid, kv, h) = scale;
+}
+
 // fp8 whole pages, one 256-thread workgroup per (page, K/V, head): the page
 // maximum over its valid tokens, then the codes (the source is read twice).
 template <int SRC>
@@ -243,8 +509,40 @@ int check_quant(const void* key, const void* value, int src_dtype, const int32_t
   return check_pool_scales(kv_dtype, pool, scales, KH, PS, D, L, P, who);
 }
 
+// The row-group kernels: their lanes cover 128 dims, load 16 source bytes and
+// store 8 code bytes at a time (every row and slice offset is a multiple of
+// those; the buffers need to start on them), and the fp8 one holds at most 32
+// tokens.
+//
+// From kManySlices (page, K/V, head) slices on, each has one wavefront (int8
+// from bf16, four / one: 2048 slices 5.5 / 6.7 us, 4096 8.3 / 9.1, 8192 14.9 /
+// 14.2, 16,384 26.0 / 22.7, 65,536 112 / 87; fp8 8192 15.7 / 13.4).
+constexpr int kManySlices = 8192;
+bool row_groups_ok(const QuantArgs& a, bool fp8) {
+  const uintptr_t src = reinterpret_cast<uintptr_t>(a.key) | reinterpret_cast<uintptr_t>(a.value);
+  return a.D <= 128 && (src & 15) == 0 && (reinterpret_cast<uintptr_t>(a.pool) & 15) == 0 && (!fp8 || a.PS <= 32);
+}
+
 template <int SRC, int DMAX>
 void launch_quant(const QuantArgs& a, int n, int kv_dtype, bool pages, hipStream_t st) {
+  if (pages && row_groups_ok(a, fp8_pool(kv_dtype))) {
+    const dim3 grid(2 * a.KH, n), slices((2 * a.KH + 3) / 4, n);
+    const bool many = (long long)n * 2 * a.KH >= kManySlices;
+    if (!fp8_pool(kv_dtype)) {
+      if (many)
+        hipLaunchKernelGGL((quant_slices_kernel<SRC, 4, false>), slices, dim3(256), 0, st, a);
+      else
+        hipLaunchKernelGGL((quant_slices_kernel<SRC, 1, false>), grid, dim3(256), 0, st, a);
+    } else if (a.PS <= 16) {
+      if (many)
+        hipLaunchKernelGGL((quant_slices_kernel<SRC, 4, true>), slices, dim3(256), 0, st, a);
+      else
+        hipLaunchKernelGGL((quant_fp8_rows_kernel<SRC, 1>), grid, dim3(256), 0, st, a);
+    } else {
+      hipLaunchKernelGGL((quant_fp8_rows_kernel<SRC, 2>), grid, dim3(256), 0, st, a);
+    }
+    return;
+  }
   if (!fp8_pool(kv_dtype)) {
     if (pages)
       hipLaunchKernelGGL((quant_i8_kernel<SRC, DMAX, true>), dim3(2 * a.KH, n, a.PS), dim3(64), 0, st, a);
