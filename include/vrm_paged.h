@@ -418,6 +418,28 @@ int vrm_topk_attend(const float* scores, int M, int N, long long ld_scores, int 
                     size_t workspace_bytes, vrm_stream_t stream);
 
 /*
+ * Both in one call over raw codes: scores of q [M][head_dim] against N
+ * compressed keys (times `scale`), the k largest of each row, and the
+ * renormalised softmax over them applied to N compressed values,
+ * out [M][head_dim] float32: KVCacheCompressor.sparse_v_attend
+ * (core/kv_quantizer.py:537-562).  The values are summed in the rotated space
+ * and rotated back once per row; they are never decompressed to memory.  Serves
+ * padded_dim 64 or 128, qjl_dim = padded_dim / 2, bits <= 4 and N <= 32768;
+ * VRM_ERR_UNSUPPORTED otherwise.  Angles aligned to 4 bytes, k_signs and
+ * workspace to 16.  workspace: >= vrm_turboquant_sparse_attend_workspace_bytes
+ * bytes (query features, scores, selection, partial sums).
+ */
+size_t vrm_turboquant_sparse_attend_workspace_bytes(int M, int N, int padded_dim, int qjl_dim);
+int vrm_turboquant_sparse_attend(const float* q, int M, const uint16_t* k_radius,
+                                 const uint8_t* k_angles, const uint8_t* k_signs,
+                                 const uint16_t* k_norms, const uint16_t* v_radius,
+                                 const uint8_t* v_angles, int N, int k, int head_dim,
+                                 int padded_dim, int n_levels, int bits, int qjl_dim,
+                                 const float* signs, const float* jl, const float* angle_lut,
+                                 float scale, void* workspace, size_t workspace_bytes, float* out,
+                                 vrm_stream_t stream);
+
+/*
  * Packed code format of KVCacheCompressor (core/kv_quantizer.py:46-105,
  * 337-371): each of `rows` rows of M uint8 values contributes the low `bits`
  * bits of every value, most significant bit first; the row's bit stream fills

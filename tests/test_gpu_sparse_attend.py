@@ -19,6 +19,7 @@ import torch
 from oracle import paged_decode as PD
 from oracle import turboquant as TQ
 from vramancer_amd import tq_pages
+from vramancer_amd.kv_quantizer import KVCacheCompressor
 from vramancer_amd.paged_attention import PagedKVCacheManager, PagedKVConfig
 from vramancer_amd.turboquant_cuda import CUDATurboQuantOps, topk_attend
 
@@ -109,6 +110,61 @@ def test_topk_attend_ties_and_negative_zero():
         torch.testing.assert_close(got.double(), _topk_reference(s, k, v), atol=1e-6, rtol=1e-6)
         kept = got > 0
         assert int(kept[0].sum()) == k and int(kept[1].sum()) == k
+
+
+@pytest.mark.parametrize("head_dim,bits,M,N,ratio", [(128, 3, 40, 4096, 0.1), (128, 4, 17, 4101, 0.2), (64, 3, 12, 2048, 0.1),
+                                                     (64, 4, 33, 16387, 0.05), (100, 2, 1, 130, 0.5), (128, 3, 70, 33, 1.0),
+                                                     (40, 1, 5, 1, 0.1), (128, 3, 16, 32768, 0.1), (128, 3, 3, 32771, 0.1)])
+def test_sparse_v_over_codes_matches_float64(head_dim, bits, M, N, ratio):
+    """sparse_v_attend on codes (the fused path up to 32,768 keys): the k
+    largest of the scores its score kernel gives, their softmax in float64
+    over the decompressed values.  Float32 sums: 1e-5 of each row's largest
+    output."""
+    _say(f"sparse over codes d{head_dim} b{bits} M{M} N{N} r{ratio}")
+    torch.manual_seed(head_dim + N)
+    comp = KVCacheCompressor(head_dim, bits).to(DEV)
+    g = torch.Generator().manual_seed(N)
+    ck, cv = (comp.compress(torch.randn(N, head_dim, generator=g).to(DEV), pack=False) for _ in range(2))
+    q = torch.randn(M, head_dim, generator=g).to(DEV)
+    got = comp.sparse_v_attend(q, ck, [cv], sparse_v_ratio=ratio)
+    args = (*comp._ops_args(), comp._hadamard_signs, comp.jl_matrix, comp.qjl_dim)
+    s = CUDATurboQuantOps.attention_score_gpu(q, ck, *args, scale=1.0 / math.sqrt(head_dim)).cpu()
+    k = max(1, math.ceil(ratio * N))
+    want = _topk_reference(s, k, comp.decompress(cv).cpu())
+    err = (got.cpu().double() - want).abs()
+    assert (err <= 1e-5 * want.abs().amax(-1, keepdim=True)).all(), f"max err {err.max():.3e}"
+    # the values in several dicts, as one per token, are the same rows
+    cut = max(1, N // 3)
+    parts = [{"radius": cv["radius"][a:b], "angles": [x[a:b] for x in cv["angles"]], "qjl_signs": cv["qjl_signs"][a:b],
+              "qjl_norms": cv["qjl_norms"][a:b], "shape": (b - a, head_dim)} for a, b in ((0, cut), (cut, N)) if b > a]
+    torch.testing.assert_close(comp.sparse_v_attend(q, ck, parts, sparse_v_ratio=ratio), got, atol=0, rtol=0)
+
+
+def test_sparse_v_ties_and_values_without_numbers():
+    """Equal keys give equal scores, of which the lowest-indexed are kept; a
+    value row with an infinite radius reaches the query rows that keep it and
+    leaves the others alone."""
+    _say("sparse ties")
+    torch.manual_seed(3)
+    comp = KVCacheCompressor(128, 3).to(DEV)
+    N, k = 500, 50
+    base = torch.randn(10, 128, generator=torch.Generator().manual_seed(1))
+    ck = comp.compress(base.repeat(N // 10, 1).to(DEV), pack=False)  # every score fifty times
+    cv = comp.compress(torch.randn(N, 128, generator=torch.Generator().manual_seed(2)).to(DEV), pack=False)
+    q = torch.randn(4, 128, generator=torch.Generator().manual_seed(4)).to(DEV)
+    args = (*comp._ops_args(), comp._hadamard_signs, comp.jl_matrix, comp.qjl_dim)
+    s = CUDATurboQuantOps.attention_score_gpu(q, ck, *args, scale=1.0 / math.sqrt(128)).cpu()
+    vals = comp.decompress(cv).cpu()
+    for keep in (k, k + 7, 3):
+        got = comp.sparse_v_attend(q, ck, [cv], sparse_v_ratio=(keep - 0.5) / N).cpu()
+        torch.testing.assert_close(got.double(), _topk_reference(s, keep, vals), atol=1e-5, rtol=1e-5)
+    order = [sorted(range(N), key=lambda n: (-float(s[m, n]), n))[:k] for m in range(4)]
+    n_bad = order[0][0]
+    cv["radius"] = cv["radius"].clone()
+    cv["radius"][n_bad] = float("inf")
+    got = comp.sparse_v_attend(q, ck, [cv], sparse_v_ratio=(k - 0.5) / N).cpu()
+    for m in range(4):
+        assert bool(torch.isfinite(got[m]).all()) == (n_bad not in order[m]), m
 
 
 def _codes(m, layer):

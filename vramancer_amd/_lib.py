@@ -72,6 +72,8 @@ SIGNATURES = {
     "vrm_kv_write": (_i, [_p, _p, _i, _p, _p, _i, _p] + [_i] * 7 + [_p]),
     "vrm_turboquant_score_workspace_bytes": (_sz, [_i, _i, _i]),
     "vrm_turboquant_score": (_i, [_p, _i, _p, _p, _p, _p] + [_i] * 6 + [_p, _p, _p, _f, _p, _sz, _p, _p]),
+    "vrm_turboquant_sparse_attend_workspace_bytes": (_sz, [_i, _i, _i, _i]),
+    "vrm_turboquant_sparse_attend": (_i, [_p, _i] + [_p] * 6 + [_i] * 7 + [_p, _p, _p, _f, _p, _sz, _p, _p]),
     "vrm_topk_attend_workspace_bytes": (_sz, [_i, _i]),
     "vrm_topk_attend": (_i, [_p, _i, _i, _ll, _i, _p, _i, _ll, _p, _ll, _p, _sz, _p]),
     "vrm_paged_decode_lse": (_i, [_p, _p, _p, _p, _p, _p, _p, _p, _sz] + [_i] * 9 + [_f, _i, _p]),

@@ -11,13 +11,16 @@
 // With k = N this is the dense softmax(s) V of the reference's k >= seq_len
 // branch.
 //
-// Selection (topk_select_kernel): the k-th largest score T of each row by a
-// radix select, four passes of 8 bits over an order-preserving integer key,
-// one workgroup per row.  S_m is every score above T plus, of the scores equal
-// to T, the lowest-indexed ones up to k in total (the reference's topk leaves
-// the choice among equal weights unspecified).  topk_attend_kernel compacts
-// S_m in index order, then computes the weights and the weighted sum.
+// Selection: the k-th largest score T of each row by a radix select over an
+// order-preserving integer key, one workgroup per row.  S_m is every score
+// above T plus, of the scores equal to T, the lowest-indexed ones up to k in
+// total (the reference's topk leaves the choice among equal weights
+// unspecified).  Rows of up to 32,768 scores are read once and stay in
+// registers through selection, weights and compaction (topk_row_kernel);
+// longer ones, and values wider than 256, take a pass over memory for every
+// step (topk_select_kernel, topk_attend_kernel).
 #include "vrm_common.h"
+#include "vrm_tq_scores.h"
 
 #include <math.h>
 
@@ -32,12 +35,6 @@ constexpr int kWaves = kThreads / 64;
 constexpr int kRowThreads = 1024;
 constexpr int kRowWaves = kRowThreads / 64;
 constexpr int kSelLoads = 8;  // scores per thread per load round of the radix select
-
-// Ascending float order <-> ascending unsigned order.
-__device__ __forceinline__ uint32_t order_key(float x) {
-  const uint32_t u = __float_as_uint(x);
-  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
 
 __global__ void __launch_bounds__(kRowThreads) topk_select_kernel(const float* scores, int N, long long ld, int k,
                                                                uint32_t* sel) {
@@ -222,6 +219,132 @@ __global__ void __launch_bounds__(kRowThreads) topk_attend_kernel(const float* s
   }
 }
 
+__device__ __forceinline__ float score_of(uint32_t key) {  // inverse of order_key
+  return __uint_as_float(key & 0x80000000u ? key ^ 0x80000000u : ~key);
+}
+
+// Selection of one row of up to kRowThreads * ITEMS scores, held as keys in
+// registers (score n = e * kRowThreads + tid in register e).  Bound: the chain
+// of barriers of three digit passes (11, 11 and 10 bits); digits this wide
+// spread ordinary scores over enough histogram bins that the LDS atomics do
+// not queue on one address, as they did on 8-bit digits (40 rows of 32,768:
+// selection 50 us -> 20).
+template <int ITEMS, bool COMPACT>
+__global__ void __launch_bounds__(kRowThreads) topk_row_kernel(const float* scores, int N, long long ld, int k,
+                                                             TopkRow* rows, int32_t* idx_ws, float* w_ws,
+                                                             RowMeta* meta) {
+  constexpr int kBins = 2048;
+  __shared__ uint32_t hist[kBins];
+  __shared__ int scan_lds[kRowWaves];
+  __shared__ float red_lds[kRowWaves];
+  __shared__ uint32_t s_bin, s_remaining, s_equal;
+  __shared__ int s_last;
+  const int tid = threadIdx.x, m = blockIdx.x;
+  const float* row = scores + (size_t)m * ld;
+  uint32_t key[ITEMS];
+  float mx = -INFINITY;
+#pragma unroll
+  for (int e = 0; e < ITEMS; ++e) {
+    const int n = e * kRowThreads + tid;
+    const float x = n < N ? row[n] : 0.f;
+    key[e] = n < N ? order_key(x) : 0u;  // below every number; k <= N, so never selected
+    if (n < N) mx = fmaxf(mx, x);
+  }
+  mx = block_max<kRowWaves>(mx, red_lds);
+  uint32_t prefix = 0, mask = 0, remaining = (uint32_t)k;
+#pragma unroll
+  for (int p = 0; p < 3; ++p) {
+    const int shift = p == 0 ? 21 : p == 1 ? 10 : 0;
+    const uint32_t digit = p == 2 ? 1023u : 2047u;
+    hist[tid] = 0;
+    hist[tid + kRowThreads] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < ITEMS; ++e)
+      if ((key[e] & mask) == prefix) atomicAdd(&hist[(key[e] >> shift) & digit], 1u);
+    __syncthreads();
+    // from the largest keys down: this thread's two bins and what lies above
+    const int b = kBins - 1 - 2 * tid;
+    const uint32_t h0 = hist[b], h1 = hist[b - 1];
+    int total;
+    const uint32_t above = (uint32_t)block_exclusive_scan<kRowWaves>((int)(h0 + h1), total, scan_lds);
+    if (above < remaining && remaining <= above + h0 + h1) {  // exactly one thread
+      const bool first = remaining <= above + h0;
+      s_bin = (uint32_t)(first ? b : b - 1);
+      s_remaining = remaining - above - (first ? 0u : h0);
+      s_equal = first ? h0 : h1;
+    }
+    __syncthreads();
+    prefix |= s_bin << shift;
+    mask |= digit << shift;
+    remaining = s_remaining;
+  }
+  // of the scores equal to T, the first `remaining` by index
+  int last_tie = N;
+  if (s_equal != remaining) {
+    int seen = 0;
+    if (tid == 0) s_last = 0;
+    for (int e = 0; e < ITEMS && seen < (int)remaining; ++e) {
+      bool eq = false;
+#pragma unroll
+      for (int i = 0; i < ITEMS; ++i) eq = i == e ? key[i] == prefix : eq;
+      const int n = e * kRowThreads + tid;
+      eq = eq && n < N;
+      int total;
+      const int rank = block_exclusive_scan<kRowWaves>(eq ? 1 : 0, total, scan_lds) + seen;
+      if (eq && rank == (int)remaining - 1) s_last = n;
+      seen += total;
+    }
+    __syncthreads();
+    last_tie = s_last;
+  }
+  if (!COMPACT) {
+    if (tid == 0) rows[m] = TopkRow{prefix, last_tie, mx, 0};
+    return;
+  }
+  int kept = 0;
+#pragma unroll
+  for (int e = 0; e < ITEMS; ++e) {
+    const int n = e * kRowThreads + tid;
+    kept += n < N && (key[e] > prefix || (key[e] == prefix && n <= last_tie)) ? 1 : 0;
+  }
+  int total;
+  int pos = block_exclusive_scan<kRowWaves>(kept, total, scan_lds);
+  int32_t* idx = idx_ws + (size_t)m * k;
+  float* wts = w_ws + (size_t)m * k;
+  float part = 0.f;
+#pragma unroll
+  for (int e = 0; e < ITEMS; ++e) {
+    const int n = e * kRowThreads + tid;
+    if (n < N && (key[e] > prefix || (key[e] == prefix && n <= last_tie)) && pos < k) {
+      const float w = expf(score_of(key[e]) - mx);
+      idx[pos] = n;
+      wts[pos] = w;
+      part += w;
+      ++pos;
+    }
+  }
+  const float l = block_sum<kRowWaves>(part, red_lds);
+  if (tid == 0) meta[m] = RowMeta{min(total, k), l};
+}
+
+template <bool COMPACT>
+void launch_rows(const float* scores, int M, int N, long long ld, int k, TopkRow* rows, int32_t* idx, float* wts,
+                 RowMeta* meta, hipStream_t st) {
+#define VRM_TOPK_ROWS(ITEMS)                                                                                  \
+  hipLaunchKernelGGL((topk_row_kernel<ITEMS, COMPACT>), dim3(M), dim3(kRowThreads), 0, st, scores, N, ld, k,  \
+                     rows, idx, wts, meta)
+  if (N <= 2 * kRowThreads)
+    VRM_TOPK_ROWS(2);
+  else if (N <= 8 * kRowThreads)
+    VRM_TOPK_ROWS(8);
+  else if (N <= 16 * kRowThreads)
+    VRM_TOPK_ROWS(16);
+  else
+    VRM_TOPK_ROWS(32);  // 64 scores a thread spill at 1024 threads
+#undef VRM_TOPK_ROWS
+}
+
 // Weighted sum of the kept values of row m = blockIdx.x, split s = blockIdx.y
 // of kSplits: the split's tokens (a contiguous range of the kept list) are
 // dealt to the wavefronts in turn, 8 tokens' loads issued together; each lane
@@ -289,6 +412,11 @@ __global__ void __launch_bounds__(kThreads) topk_combine_kernel(const float* par
 }
 
 }  // namespace
+
+void launch_topk_select(const float* scores, int M, int N, long long ld, int k, TopkRow* rows, hipStream_t st) {
+  launch_rows<false>(scores, M, N, ld, k, rows, nullptr, nullptr, nullptr, st);
+}
+
 }  // namespace vrm
 
 using namespace vrm;
@@ -349,9 +477,13 @@ extern "C" int vrm_topk_attend(const float* scores, int M, int N, long long ld_s
   RowMeta* meta = reinterpret_cast<RowMeta*>(ws + meta_off);
   float* part = reinterpret_cast<float*>(ws + part_off);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(topk_select_kernel, dim3(M), dim3(kRowThreads), 0, st, scores, N, ld_scores, k, sel);
-  hipLaunchKernelGGL(topk_attend_kernel, dim3(M), dim3(kRowThreads), 0, st, scores, N, ld_scores, k, sel, values, D,
-                     ld_values, idx, wts, meta, out, ld_out);
+  if (N <= kMaxSelectRow && D <= kMaxFastD) {
+    launch_rows<true>(scores, M, N, ld_scores, k, nullptr, idx, wts, meta, st);
+  } else {
+    hipLaunchKernelGGL(topk_select_kernel, dim3(M), dim3(kRowThreads), 0, st, scores, N, ld_scores, k, sel);
+    hipLaunchKernelGGL(topk_attend_kernel, dim3(M), dim3(kRowThreads), 0, st, scores, N, ld_scores, k, sel, values, D,
+                       ld_values, idx, wts, meta, out, ld_out);
+  }
   if (D <= kMaxFastD) {
     hipLaunchKernelGGL(topk_pv_kernel, dim3(M, kSplits), dim3(kThreads), 0, st, idx, wts, meta, k, values, D,
                        ld_values, part);

@@ -222,27 +222,34 @@ class KVCacheCompressor(nn.Module):
         if scale is None:
             scale = 1.0 / math.sqrt(self.head_dim)
         compressed_k = self._unpack_compressed(compressed_k)
-        scores = CUDATurboQuantOps.attention_score_gpu(
-            q, compressed_k, *self._ops_args(), self._hadamard_signs, self.jl_matrix, self.qjl_dim, scale=scale)
+        args = (*self._ops_args(), self._hadamard_signs, self.jl_matrix, self.qjl_dim)
+        values = self._merge_rows(compressed_v_list)
+        out = CUDATurboQuantOps.sparse_attend_gpu(q, compressed_k, values, sparse_v_ratio, scale, *args)
+        if out is not None:
+            return out
+        scores = CUDATurboQuantOps.attention_score_gpu(q, compressed_k, *args, scale=scale)
         seq_len = scores.shape[-1]
         k = max(1, int(math.ceil(sparse_v_ratio * seq_len)))
-        v_mat = self._decompress_list(compressed_v_list)
+        v_mat = CUDATurboQuantOps.decompress_gpu(values, *self._ops_args(), self._hadamard_signs)
         if v_mat.shape[0] != seq_len:
             raise RuntimeError(f"{v_mat.shape[0]} value rows for {seq_len} keys")
         return topk_attend(scores, min(k, seq_len), v_mat)
 
-    def _decompress_list(self, compressed_list):
-        """Rows of every dict of the list, decompressed in one launch: [rows, head_dim]."""
+    def _merge_rows(self, compressed_list):
+        """Radii and angles of every dict of the list as one; a single dict's
+        arrays are used as they are."""
         parts = [self._unpack_compressed(c) for c in compressed_list]
         if not parts:
             raise RuntimeError("empty value list")
-        merged = {
-            "radius": torch.cat([c["radius"].reshape(-1) for c in parts]),
-            "angles": [torch.cat([c["angles"][l].reshape(-1, c["angles"][l].shape[-1]) for c in parts])
-                       for l in range(len(parts[0]["angles"]))],
-        }
+        levels = range(len(parts[0]["angles"]))
+        radii = [c["radius"].reshape(-1) for c in parts]
+        angles = [[c["angles"][l].reshape(-1, c["angles"][l].shape[-1]) for c in parts] for l in levels]
+        if len(parts) == 1:
+            merged = {"radius": radii[0], "angles": [a[0] for a in angles]}
+        else:
+            merged = {"radius": torch.cat(radii), "angles": [torch.cat(a) for a in angles]}
         merged["shape"] = (merged["radius"].shape[0], self.head_dim)
-        return CUDATurboQuantOps.decompress_gpu(merged, *self._ops_args(), self._hadamard_signs)
+        return merged
 
     def bits_per_dim(self):
         """((padded_dim - 1) * bits + 16 + qjl_dim + 16) / head_dim."""

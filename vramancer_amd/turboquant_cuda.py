@@ -302,6 +302,50 @@ class CUDATurboQuantOps:
         _lib.check(rc, "turboquant attention_score")
         return scores
 
+    @staticmethod
+    def sparse_attend_gpu(q, compressed_k: dict, values: dict, ratio: float, scale: float, head_dim: int,
+                          padded_dim: int, n_levels: int, bits_per_angle: int, hadamard_signs, jl_matrix,
+                          qjl_dim: int):
+        """Sparse V over raw codes, [n_queries, head_dim] float32: scores,
+        top max(1, ceil(ratio * N)) of each row and their weighted values
+        without decompressing them; None for settings and arrays the fused
+        path does not serve."""
+        import torch
+
+        if (padded_dim not in (64, 128) or bits_per_angle > 4 or qjl_dim != padded_dim // 2 or not q.is_cuda
+                or jl_matrix.shape != (qjl_dim, padded_dim) or hadamard_signs.shape != (padded_dim,)):
+            return None
+        device = q.device
+        flat_q = q.reshape(-1, head_dim).float().contiguous()
+        k_radius = compressed_k["radius"].reshape(-1).to(torch.float16).contiguous()
+        k_angles = level_bins(compressed_k["angles"], padded_dim - 1)
+        k_signs = compressed_k["qjl_signs"].to(torch.uint8).contiguous()
+        k_norms = compressed_k["qjl_norms"].reshape(-1).to(torch.float16).contiguous()
+        v_radius = values["radius"].to(torch.float16).contiguous()
+        v_angles = level_bins(values["angles"], padded_dim - 1)
+        M, N = flat_q.shape[0], k_radius.shape[0]
+        if (not 1 <= M <= 65535 or not 1 <= N <= 32768 or k_angles.shape != (N, padded_dim - 1)
+                or k_signs.shape != (N, qjl_dim) or k_norms.shape != (N,) or v_radius.shape != (N,)
+                or v_angles.shape != (N, padded_dim - 1)
+                or any(t.device != device for t in (k_radius, k_angles, k_signs, k_norms, v_radius, v_angles))
+                or k_angles.data_ptr() % 4 or v_angles.data_ptr() % 4 or k_signs.data_ptr() % 16):
+            return None
+        k = min(max(1, int(math.ceil(ratio * N))), N)
+        signs_f = hadamard_signs.to(device=device, dtype=torch.float32).contiguous()
+        jl_f = jl_matrix.to(device=device, dtype=torch.float32).contiguous()
+        lib = _lib.load()
+        ws = torch.empty(lib.vrm_turboquant_sparse_attend_workspace_bytes(M, N, padded_dim, qjl_dim),
+                         dtype=torch.uint8, device=device)
+        out = torch.empty((M, head_dim), dtype=torch.float32, device=device)
+        rc = lib.vrm_turboquant_sparse_attend(
+            _lib.ptr(flat_q), M, _lib.ptr(k_radius), _lib.ptr(k_angles), _lib.ptr(k_signs), _lib.ptr(k_norms),
+            _lib.ptr(v_radius), _lib.ptr(v_angles), N, k, head_dim, padded_dim, n_levels, bits_per_angle, qjl_dim,
+            _lib.ptr(signs_f), _lib.ptr(jl_f), _lib.ptr(angle_lut(bits_per_angle, device)), float(scale),
+            _lib.ptr(ws), ws.numel(), _lib.ptr(out), _lib.stream_of(flat_q),
+        )
+        _lib.check(rc, "turboquant sparse_attend")
+        return out
+
 
 def topk_attend(scores, k: int, values):
     """Renormalised top-k softmax attention: for each row of ``scores`` [M, N]
