@@ -18,43 +18,78 @@ int launch_status(const char* what);
 
 constexpr int kWave = 64;
 
-// Butterfly exchange across lanes lane ^ mask of a 64-wide wavefront.
-// ds_swizzle covers masks below 32 within each 32-lane half; mask 32 crosses
-// halves and uses ds_bpermute.
+// Butterfly exchange across lanes lane ^ mask of a 64-wide wavefront, on the
+// vector ALU throughout: DPP within a row of 16 lanes, v_permlane swaps across
+// rows.  (The LDS exchange unit, ds_swizzle / ds_bpermute, answers after some
+// 100 cycles, and these sit on dependency chains: in the decode two of them
+// per page pair, between the scores and the weights.  Small decodes take 1 us
+// less, float32 pools 12 %, and the shared-items pass 9 registers less.)
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+
 template <int MASK>
 __device__ __forceinline__ float xor_shfl(float v) {
   static_assert(MASK > 0 && MASK < 64 && (MASK & (MASK - 1)) == 0, "power-of-two mask");
-  if constexpr (MASK < 32) {
-    // ds_swizzle bit mode: and_mask = 0x1f, or_mask = 0, xor_mask = MASK.
-    constexpr int pattern = 0x1f | (MASK << 10);
-    return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), pattern));
-  } else {
-    const int lane = __lane_id();
-    return __int_as_float(__builtin_amdgcn_ds_bpermute((lane ^ MASK) << 2, __float_as_int(v)));
+  if constexpr (MASK == 1) return dpp<0xb1>(v);              // quad_perm 1, 0, 3, 2
+  if constexpr (MASK == 2) return dpp<0x4e>(v);              // quad_perm 2, 3, 0, 1
+  if constexpr (MASK == 4) return dpp<0x1b>(dpp<0x141>(v));  // lane ^ 7 (row_half_mirror), then ^ 3
+  if constexpr (MASK == 8) return dpp<0x128>(v);             // row_ror 8
+  if constexpr (MASK == 16) {  // the swap leaves {even rows twice}, {odd rows twice}
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float((__lane_id() & 16) ? r[0] : r[1]);
   }
+  if constexpr (MASK == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float((__lane_id() & 32) ? r[0] : r[1]);
+  }
+}
+
+// v op (v of lane ^ MASK): across rows the two results of the swap are the
+// two operands, so nothing needs selecting.
+template <int MASK, typename Op>
+__device__ __forceinline__ float xor_reduce(float v, Op op) {
+  if constexpr (MASK == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  } else if constexpr (MASK == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  } else {
+    return op(v, xor_shfl<MASK>(v));
+  }
+}
+template <int MASK>
+__device__ __forceinline__ float xor_add(float v) {
+  return xor_reduce<MASK>(v, [](float a, float b) { return a + b; });
+}
+template <int MASK>
+__device__ __forceinline__ float xor_max(float v) {
+  return xor_reduce<MASK>(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // Sum over the aligned group of N lanes (N a power of two <= 64) that
 // contains this lane; every lane of the group receives the total.
 template <int N>
 __device__ __forceinline__ float group_sum(float v) {
-  if constexpr (N >= 2) v += xor_shfl<1>(v);
-  if constexpr (N >= 4) v += xor_shfl<2>(v);
-  if constexpr (N >= 8) v += xor_shfl<4>(v);
-  if constexpr (N >= 16) v += xor_shfl<8>(v);
-  if constexpr (N >= 32) v += xor_shfl<16>(v);
-  if constexpr (N >= 64) v += xor_shfl<32>(v);
+  if constexpr (N >= 2) v = xor_add<1>(v);
+  if constexpr (N >= 4) v = xor_add<2>(v);
+  if constexpr (N >= 8) v = xor_add<4>(v);
+  if constexpr (N >= 16) v = xor_add<8>(v);
+  if constexpr (N >= 32) v = xor_add<16>(v);
+  if constexpr (N >= 64) v = xor_add<32>(v);
   return v;
 }
 
 template <int N>
 __device__ __forceinline__ float group_max(float v) {
-  if constexpr (N >= 2) v = fmaxf(v, xor_shfl<1>(v));
-  if constexpr (N >= 4) v = fmaxf(v, xor_shfl<2>(v));
-  if constexpr (N >= 8) v = fmaxf(v, xor_shfl<4>(v));
-  if constexpr (N >= 16) v = fmaxf(v, xor_shfl<8>(v));
-  if constexpr (N >= 32) v = fmaxf(v, xor_shfl<16>(v));
-  if constexpr (N >= 64) v = fmaxf(v, xor_shfl<32>(v));
+  if constexpr (N >= 2) v = xor_max<1>(v);
+  if constexpr (N >= 4) v = xor_max<2>(v);
+  if constexpr (N >= 8) v = xor_max<4>(v);
+  if constexpr (N >= 16) v = xor_max<8>(v);
+  if constexpr (N >= 32) v = xor_max<16>(v);
+  if constexpr (N >= 64) v = xor_max<32>(v);
   return v;
 }
 
@@ -62,12 +97,12 @@ __device__ __forceinline__ float group_max(float v) {
 // STRIDE, 2*STRIDE, ..., 32.
 template <int STRIDE>
 __device__ __forceinline__ float strided_sum(float v) {
-  if constexpr (STRIDE <= 1) v += xor_shfl<1>(v);
-  if constexpr (STRIDE <= 2) v += xor_shfl<2>(v);
-  if constexpr (STRIDE <= 4) v += xor_shfl<4>(v);
-  if constexpr (STRIDE <= 8) v += xor_shfl<8>(v);
-  if constexpr (STRIDE <= 16) v += xor_shfl<16>(v);
-  if constexpr (STRIDE <= 32) v += xor_shfl<32>(v);
+  if constexpr (STRIDE <= 1) v = xor_add<1>(v);
+  if constexpr (STRIDE <= 2) v = xor_add<2>(v);
+  if constexpr (STRIDE <= 4) v = xor_add<4>(v);
+  if constexpr (STRIDE <= 8) v = xor_add<8>(v);
+  if constexpr (STRIDE <= 16) v = xor_add<16>(v);
+  if constexpr (STRIDE <= 32) v = xor_add<32>(v);
   return v;
 }
 

@@ -87,26 +87,29 @@ __device__ __forceinline__ int seq_pages(int ctx, int max_pp, int ps = kPS) {
   return ctx > 0 ? min((ctx + ps - 1) / ps, max_pp) : 0;
 }
 
-__device__ __forceinline__ int wave_sum_int(int v) {
-#pragma unroll
-  for (int m = 1; m < 64; m <<= 1) v += __builtin_amdgcn_ds_bpermute((__lane_id() ^ m) << 2, v);
-  return v;
+// Whole-wavefront scan, sum and maximum on DPP: sums within rows of 16 lanes
+// (row_shr 1, 2, 4, 8, zeros shifted in), then the rows' totals (row_bcast 15
+// into rows 1 and 3, row_bcast 31 into rows 2 and 3).
+__device__ __forceinline__ int wave_inclusive_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+  return x;
 }
 
-__device__ __forceinline__ int wave_max_int(int v) {
-#pragma unroll
-  for (int m = 1; m < 64; m <<= 1) v = max(v, __builtin_amdgcn_ds_bpermute((__lane_id() ^ m) << 2, v));
-  return v;
-}
+__device__ __forceinline__ int wave_sum_int(int v) { return __builtin_amdgcn_readlane(wave_inclusive_scan(v), 63); }
 
-__device__ __forceinline__ int wave_inclusive_scan(int v) {
-  const int lane = __lane_id();
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int t = __builtin_amdgcn_ds_bpermute(max(lane - d, 0) << 2, v);
-    if (lane >= d) v += t;
-  }
-  return v;
+__device__ __forceinline__ int wave_max_int(int x) {  // lanes without a source keep their own value
+  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x111, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x112, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x114, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x118, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x142, 0xa, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x143, 0xc, 0xf, false));
+  return __builtin_amdgcn_readlane(x, 63);
 }
 
 // Finds work item `item` of the batch.  Every wave of a launch derives the

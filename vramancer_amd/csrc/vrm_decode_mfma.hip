@@ -515,8 +515,8 @@ __device__ __forceinline__ int stream_item(const DecodeArgs& a, int G, const int
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) qmax = fmaxf(qmax, fabsf(qv[j][e]));
-    qmax = fmaxf(qmax, xor_shfl<16>(qmax));
-    qmax = fmaxf(qmax, xor_shfl<32>(qmax));
+    qmax = xor_max<16>(qmax);
+    qmax = xor_max<32>(qmax);
     const float inv = qmax > 0.f ? 127.f / qmax : 0.f;
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
@@ -665,8 +665,8 @@ __device__ __forceinline__ int stream_item(const DecodeArgs& a, int G, const int
     }
     int e_new = vexp;
     if (__builtin_amdgcn_ballot_w64(vm > vlimit) != 0) {
-      float wm = fmaxf(vm, xor_shfl<16>(vm));
-      wm = fmaxf(wm, xor_shfl<32>(wm));
+      float wm = xor_max<16>(vm);
+      wm = xor_max<32>(wm);
       if (wm <= 3.0e38f) {  // finite: an inf scale keeps e (its tokens give inf / NaN as in the reference)
         int ex;
         (void)frexpf(wm, &ex);  // wm < 2^ex
@@ -677,8 +677,8 @@ __device__ __forceinline__ int stream_item(const DecodeArgs& a, int G, const int
     float pm = sc[0];
 #pragma unroll
     for (int r = 1; r < 8; ++r) pm = fmaxf(pm, sc[r]);
-    pm = fmaxf(pm, xor_shfl<16>(pm));
-    pm = fmaxf(pm, xor_shfl<32>(pm));
+    pm = xor_max<16>(pm);
+    pm = xor_max<32>(pm);
     const bool up = pm > m_run + kLazyRescale;
     if (up || e_new != vexp) {
       const float m_new = up ? pm : m_run;
@@ -764,8 +764,8 @@ __device__ __forceinline__ int stream_item(const DecodeArgs& a, int G, const int
     a.out[((size_t)b * a.H + h0) * D + lane] = __uint_as_float(probe);  // lane < 64 <= D
     return batch_items;
   }
-  float l_tot = l_run + xor_shfl<16>(l_run);
-  l_tot += xor_shfl<32>(l_tot);
+  float l_tot = xor_add<16>(l_run);
+  l_tot = xor_add<32>(l_tot);
   if constexpr (BALANCED) {
     // an item that is its whole sequence goes straight to out when the call
     // has one (the merge pass then leaves that sequence alone)
@@ -1035,8 +1035,8 @@ __global__ void __launch_bounds__(64 * kMaxWaves) decode_stream_float_kernel(Dec
     float pm = sc[0];
 #pragma unroll
     for (int r = 1; r < 8; ++r) pm = fmaxf(pm, sc[r]);
-    pm = fmaxf(pm, xor_shfl<16>(pm));
-    pm = fmaxf(pm, xor_shfl<32>(pm));
+    pm = xor_max<16>(pm);
+    pm = xor_max<32>(pm);
     if (pm > m_run + kLazyRescale) {
       const float alpha = __builtin_amdgcn_exp2f(m_run - pm);
       l_run *= alpha;
@@ -1087,8 +1087,8 @@ __global__ void __launch_bounds__(64 * kMaxWaves) decode_stream_float_kernel(Dec
     }
   }
 
-  float l_tot = l_run + xor_shfl<16>(l_run);
-  l_tot += xor_shfl<32>(l_tot);
+  float l_tot = xor_add<16>(l_run);
+  l_tot = xor_add<32>(l_tot);
   if (col < G) {
     float* out = a.part_acc + ((size_t)item * a.H + h0 + col) * D;
 #pragma unroll
@@ -1227,12 +1227,12 @@ __global__ void __launch_bounds__(64 * kMaxWaves) decode_stream_q4_kernel(Decode
       qmax = fmaxf(qmax, fabsf(qv[c][o]));
       s += qv[c][o] * a.qscale;
     }
-    s += xor_shfl<16>(s);
-    s += xor_shfl<32>(s);
+    s = xor_add<16>(s);
+    s = xor_add<32>(s);
     qsum[c] = s;
   }
-  qmax = fmaxf(qmax, xor_shfl<16>(qmax));
-  qmax = fmaxf(qmax, xor_shfl<32>(qmax));
+  qmax = xor_max<16>(qmax);
+  qmax = xor_max<32>(qmax);
   const float inv = qmax > 0.f ? 127.f / qmax : 0.f;
   const float qunit = qmax * (1.f / 127.f) * a.qscale * kInv254;  // per unit of 254 d1 + d2 + d3 / 254
   // the zero points' share in the same units: -sum_{d in g} q_d / qunit
@@ -1374,12 +1374,12 @@ __global__ void __launch_bounds__(64 * kMaxWaves) decode_stream_q4_kernel(Decode
           vm = fmaxf(vm, fmaxf((float)h[0], (float)h[1]));
         }
       }
-      float wm = fmaxf(vm, xor_shfl<1>(vm));
-      wm = fmaxf(wm, xor_shfl<2>(wm));
-      wm = fmaxf(wm, xor_shfl<4>(wm));
-      wm = fmaxf(wm, xor_shfl<8>(wm));
-      wm = fmaxf(wm, xor_shfl<16>(wm));
-      wm = fmaxf(wm, xor_shfl<32>(wm));
+      float wm = xor_max<1>(vm);
+      wm = xor_max<2>(wm);
+      wm = xor_max<4>(wm);
+      wm = xor_max<8>(wm);
+      wm = xor_max<16>(wm);
+      wm = xor_max<32>(wm);
       if (wm <= 65504.f) {  // finite: an inf scale keeps e (its tokens give inf / NaN as in the reference)
         int ex;
         (void)frexpf(wm, &ex);  // wm < 2^ex
@@ -1398,8 +1398,8 @@ __global__ void __launch_bounds__(64 * kMaxWaves) decode_stream_q4_kernel(Decode
     float pm = sc[0];
 #pragma unroll
     for (int r = 1; r < 8; ++r) pm = fmaxf(pm, sc[r]);
-    pm = fmaxf(pm, xor_shfl<16>(pm));
-    pm = fmaxf(pm, xor_shfl<32>(pm));
+    pm = xor_max<16>(pm);
+    pm = xor_max<32>(pm);
     const bool up = pm > m_run + kLazyRescale;
     if (up || e_new != vexp) {
       const float m_new = up ? pm : m_run;
@@ -1472,13 +1472,13 @@ __global__ void __launch_bounds__(64 * kMaxWaves) decode_stream_q4_kernel(Decode
     }
   }
 
-  float l_tot = l_run + xor_shfl<16>(l_run);
-  l_tot += xor_shfl<32>(l_tot);
+  float l_tot = xor_add<16>(l_run);
+  l_tot = xor_add<32>(l_tot);
   float corr_tot[NG];
 #pragma unroll
   for (int g = 0; g < NG; ++g) {
-    corr_tot[g] = corr[g] + xor_shfl<16>(corr[g]);
-    corr_tot[g] += xor_shfl<32>(corr_tot[g]);
+    corr_tot[g] = xor_add<16>(corr[g]);
+    corr_tot[g] = xor_add<32>(corr_tot[g]);
   }
   if (col < G) {
     float* out = a.part_acc + ((size_t)item * a.H + h0 + col) * D;
@@ -1495,6 +1495,18 @@ __global__ void __launch_bounds__(64 * kMaxWaves) decode_stream_q4_kernel(Decode
   }
 }
 
+// LDS a float-stream workgroup of W wavefronts asks for (and leaves unused) to
+// hold the kernel at two wavefronts per SIMD where its registers would allow
+// three: at head_dim 112 and 128 the pool's reads run slower with more bytes
+// in flight (32 sequences of 1k-8k tokens, 28 / 4 heads of 128, bf16: 69.2 us
+// with two, 73.8 with three; 64 of 4k, 40 / 8 heads of 112: 182 against 198).
+// Narrower heads are faster with the three or four that fit.
+size_t float_stream_lds(int D, int W) {
+  if (D < 112) return 0;
+  const size_t share = (size_t)160 * 1024 / (8 / W);  // 8 wavefronts on a CU's four SIMDs
+  return share < 64 * 1024 ? share : 64 * 1024;
+}
+
 template <int KIND, int D>
 void launch_kernel(const DecodeArgs& a0, int B, int units, int W, int G, hipStream_t st) {
   const void* fn;
@@ -1504,8 +1516,9 @@ void launch_kernel(const DecodeArgs& a0, int B, int units, int W, int G, hipStre
     fn = reinterpret_cast<const void*>(&decode_stream_q4_kernel);
   else
     fn = reinterpret_cast<const void*>(&decode_stream_float_kernel<KIND, D <= 128 ? D : 128>);
+  const size_t lds = KIND == K_BF16 || KIND == K_F16 ? float_stream_lds(D, W) : 0;
   DecodeArgs a = a0;
-  a.target = items_target(fn, W, 0, units);
+  a.target = items_target(fn, W, lds, units);
   dim3 grid(B + 2 * a.target, units / W, 1);  // at most B + 2 target work items
   dim3 block(64 * W);
   if constexpr (KIND == K_I8 || KIND == K_FP8)
@@ -1513,7 +1526,7 @@ void launch_kernel(const DecodeArgs& a0, int B, int units, int W, int G, hipStre
   else if constexpr (KIND == K_Q4)
     hipLaunchKernelGGL(decode_stream_q4_kernel, grid, block, 0, st, a, G);
   else if constexpr (D <= 128)
-    hipLaunchKernelGGL((decode_stream_float_kernel<KIND, D>), grid, block, 0, st, a, G);
+    hipLaunchKernelGGL((decode_stream_float_kernel<KIND, D>), grid, block, lds, st, a, G);
 }
 
 template <int KIND>

@@ -749,8 +749,8 @@ __global__ void __launch_bounds__(64 * (WIDE ? kWideWaves : kWaves), WIDE ? 1 : 
         // hi column + lo column of head hcol
         qb[col][QS * (2 * h + (row >> 3)) + 8 * c + (row & 7)] = acc[2 * c + h][r] + row_swap8(acc[2 * c + h][r]);
       }
-  float l_tot = l_run + xor_shfl<16>(l_run);
-  l_tot += xor_shfl<32>(l_tot);
+  float l_tot = xor_add<16>(l_run);
+  l_tot = xor_add<32>(l_tot);
   wave_sync();
   float sg[PER];
 #pragma unroll

@@ -257,12 +257,12 @@ __global__ void __launch_bounds__(512) tq_encode_tile_kernel(TqEncodeArgs a, int
         }
       }
       bool e;
-      float o = other16(child[0]);
+      float o = xor_shfl<16>(child[0]);
       float x0 = g & 1 ? o : child[0], x1 = g & 1 ? child[0] : o;
       bin_a = (uint32_t)vrm_tq_bin::fast_bin<BITS, false>(x0, x1, __builtin_amdgcn_rcpf(fmaxf(x0, x1)), e);
       edge = edge || e;
       const float half = radius_of(x0, x1);
-      o = other32(half);
+      o = xor_shfl<32>(half);
       x0 = g & 2 ? o : half;
       x1 = g & 2 ? half : o;
       bin_b = (uint32_t)vrm_tq_bin::fast_bin<BITS, false>(x0, x1, __builtin_amdgcn_rcpf(fmaxf(x0, x1)), e);
@@ -415,8 +415,8 @@ __global__ void __launch_bounds__(512) tq_encode_tile_kernel(TqEncodeArgs a, int
 #pragma unroll
       for (int k = 0; k < QJL / 32; ++k) {
         uint32_t x32 = (((pos >> (8 * k)) & 15u) << (4 * g)) | (((pos >> (8 * k + 4)) & 15u) << (16 + 4 * g));
-        x32 |= __float_as_uint(other16(__uint_as_float(x32)));
-        x32 |= __float_as_uint(other32(__uint_as_float(x32)));
+        x32 |= __float_as_uint(xor_shfl<16>(__uint_as_float(x32)));
+        x32 |= __float_as_uint(xor_shfl<32>(__uint_as_float(x32)));
         words[k] = x32;
       }
       sign_word = QJL == 32 || g == 0 ? words[0] : words[QJL / 32 - 1];

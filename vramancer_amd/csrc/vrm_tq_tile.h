@@ -12,16 +12,6 @@ namespace {
 
 constexpr int kTile = 16;  // rows per wavefront
 
-// Value of the lane 16 (32) lanes away: neighbour quarters, then halves.
-__device__ __forceinline__ float other16(float v) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float((__lane_id() & 16) ? r[0] : r[1]);
-}
-__device__ __forceinline__ float other32(float v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float((__lane_id() & 32) ? r[0] : r[1]);
-}
-
 // One butterfly stage across lanes for two elements a, b: the lower lane
 // keeps lower + upper, the upper lane lower - upper.  The swap gathers both
 // lanes' operands of a in the lower lane and of b in the upper one.
