@@ -252,6 +252,37 @@ def test_shared_items_many_sequences(dtype, H, KH, D):
     assert not out[torch.tensor(ctxs) == 0].any(), "empty sequences give zero rows"
 
 
+@pytest.mark.parametrize("dtype", [torch.int8, torch.float8_e4m3fn], ids=["int8", "fp8"])
+@pytest.mark.parametrize("H,KH,D", [(40, 8, 128), (12, 12, 64), (14, 2, 96), (64, 2, 80)])
+def test_routes_of_a_quantized_batch(dtype, H, KH, D):
+    """The same ragged batches (an empty sequence, a page's edges, one long
+    sequence) under page tables as wide as the longest sequence, 90, 200 and
+    700 pages: balanced workgroups of one unit (and of two, with 40
+    sequences), work items and shared rows, by the table's width.  Every
+    output and log-sum-exp matches the oracle's and the other routes'."""
+    _say(f"routes {dtype} H{H} KH{KH} D{D}")
+    g = torch.Generator().manual_seed(H + D)
+    for ctxs in ([533], [1, 16, 0, 17, 700, 15, 64, 33], [int(x) for x in torch.randint(1, 500, (40,), generator=g)]):
+        outs, lses = [], []
+        for width in (0, 90, 200, 700):
+            longest = (max(ctxs) + 15) // 16
+            q, pool, sc, table, lens = _pool_case(dtype, len(ctxs), H, KH, D, ctxs, seed=H + D,
+                                                  table_pad=max(0, width - longest))
+            d = [t.to(DEV) for t in (q, pool, sc, table, lens)]
+            lse = torch.full((len(ctxs), H), float("nan"), device=DEV)
+            out = paged_attention_decode(d[0], d[1], d[3], d[4], 1, kv_scales=d[2])
+            out2 = paged_attention_decode(d[0], d[1], d[3], d[4], 1, kv_scales=d[2], lse=lse)
+            _assert_rerun(out, out2, True, f"lse call, width {width}")
+            outs.append(out)
+            lses.append(lse)
+        ref = PD.paged_attention_decode(q, pool, table, lens, 1, kv_scales=sc)
+        for out, lse in zip(outs, lses):
+            _assert_close(out, ref, f"{len(ctxs)} sequences")
+            _assert_rerun(out, outs[0], True, "routes")
+            # -inf where a sequence is empty; else float32 rounding of a sum of up to 700 terms
+            torch.testing.assert_close(lse, lses[0], atol=1e-5, rtol=1e-6)
+
+
 @pytest.mark.parametrize("H,KH,D", [(16, 4, 128), (40, 8, 128), (12, 2, 128), (14, 2, 128), (10, 2, 64),
                                     (12, 2, 256)])
 def test_decode_q4_matches_oracle(H, KH, D):

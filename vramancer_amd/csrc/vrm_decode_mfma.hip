@@ -834,8 +834,8 @@ __device__ __forceinline__ DecodeArgs kernel_args_afresh() {
 template <int KIND, int D, bool BALANCED, bool LOADS = false, bool ITEMS = false, int UPW = kUnitsPerWg>
 __global__ void __launch_bounds__(64 * (BALANCED ? kMaxBalancedWaves : kMaxWaves))
     decode_stream_kernel(DecodeArgs a, int G) {
-  static_assert(UPW == kUnitsPerWg || (ITEMS && UPW <= kMaxUnitsPerWg && kMaxBalancedWaves % UPW == 0),
-                "only the shared-items pass takes other unit counts");
+  static_assert(UPW == kUnitsPerWg || (BALANCED && !LOADS && UPW <= kMaxUnitsPerWg && kMaxBalancedWaves % UPW == 0),
+                "only balanced builds that compute take other unit counts");
   if constexpr (ITEMS) {
     for (int item = 0, items = 1; item < items; ++item) {
       const DecodeArgs ai = kernel_args_afresh();
@@ -1556,6 +1556,16 @@ hipError_t launch_balanced_d(const DecodeArgs& a, int B, int G, hipStream_t st) 
   // the launch shape of the decode itself, for both builds
   const void* fn = reinterpret_cast<const void*>(&decode_stream_kernel<KIND, D, true, false>);
   const int resident = items_target(fn, kMaxBalancedWaves, 0, 1);  // resident waves (capped)
+  // one unit per workgroup while that fills no more than the resident round:
+  // all 12 wavefronts then share one kv-head's pages
+  if constexpr (!LOADS) {
+    const size_t lds = balanced_lds_bytes(a.max_pp, kMaxBalancedWaves, G, D);
+    if ((long)B * units * kMaxBalancedWaves <= resident && lds <= kMaxBalancedLds) {
+      hipLaunchKernelGGL((decode_stream_kernel<KIND, D, true, false, false, 1>), dim3(B, units, 1),
+                         dim3(64 * kMaxBalancedWaves), lds, st, a, G);
+      return hipGetLastError();
+    }
+  }
   for (int wpu = 6; wpu >= 1; wpu = wpu == 6 ? 4 : wpu / 2) {
     const int W = kUnitsPerWg * wpu;
     const size_t lds = balanced_lds_bytes(a.max_pp, W, G, D);

@@ -704,6 +704,35 @@ int check_kind_shape(int kind, int D, int PS, const char* who) {
   return VRM_OK;
 }
 
+// How an int8 / fp8 batch that the shared-items pass could take is decoded,
+// from what the host knows: sequences, (kv-head, head chunk) units and the
+// page table's width, the longest a sequence can be.
+//   balanced: one workgroup per sequence and unit (or two), one launch, time
+//     by the longest sequence;
+//   items: 4 pages or more per wavefront and a merge launch, for few pages;
+//   shared: rows of equal page counts and a merge launch, for the rest.
+// The times are fits to 576 batches (1 to 128 sequences of 64 to 65,536
+// tokens, equal and drawn from an eighth of the longest up, 40 / 8 and 28 / 4
+// heads of 128 and 12 / 12 of 64): a workgroup's 9.3 us and 0.08 us per page of
+// 128 dims (all 12 wavefronts on one unit; twice that with two units, from 256
+// workgroups on), against 13 us and 0.52 ns per page and unit.  The slack of
+// 1 to 2.5 us, and 256 pages at most, keep a table that is wider than its
+// sequences from costing more than the shared rows would have.  Over those
+// batches the choice takes 0.63 of the shared rows' time (128 sequences of up
+// to 64 tokens 86.7 -> 10.2 us, 8 of up to 2048 26.5 -> 17.9, 64 of up to 4096
+// 75.7 -> 69.0); where a batch loses, it loses at most 6 %.
+enum class QuantPass { kBalanced, kItems, kShared };
+QuantPass quant_pass(int B, int units, int max_pp, int D) {
+  const double wgs = (double)B * units, work = wgs * max_pp;
+  const double page = 0.018 + 0.00049 * D;
+  const double balanced = 9.3 + (wgs <= 256 ? page * max_pp : 2 * page * max_pp * (wgs > 512 ? wgs / 512 : 1.0));
+  const double items = 13.0 + 0.00052 * work * (D / 128.0);
+  const double slack = B == 1 ? 1.0 : D >= 96 ? 2.5 : 1.5;
+  if (max_pp <= (wgs <= 512 ? 256 : 128) && balanced <= items + slack) return QuantPass::kBalanced;
+  if (work <= 4096 && (B > 1 || D >= 96)) return QuantPass::kItems;
+  return QuantPass::kShared;
+}
+
 int run_decode(DecodeArgs a, int kind, float* out, void* workspace, size_t workspace_bytes, int B, int D, int PS,
                float scale, hipStream_t st, int passes) {
   // The matrix-core stream kernels take the int8 / fp8 pools at every
@@ -734,10 +763,12 @@ int run_decode(DecodeArgs a, int kind, float* out, void* workspace, size_t works
   // int8 / fp8 at page 16 and head_dim 64 .. 128: the work items' pages are
   // shared by balanced workgroups (12 wavefronts, page pairs handed out in
   // LDS), when the page table fits their LDS copy
-  const bool shared = (kind == K_I8 || kind == K_FP8) && PS == kPS && D >= 64 && D <= 128 && D % 16 == 0 &&
-                      balanced_lds_bytes(a.max_pp, kMaxBalancedWaves, G, D) <= shared_items_max_lds();
+  const bool shared_ok = (kind == K_I8 || kind == K_FP8) && PS == kPS && D >= 64 && D <= 128 && D % 16 == 0 &&
+                         balanced_lds_bytes(a.max_pp, kMaxBalancedWaves, G, D) <= shared_items_max_lds();
   const int units = a.KH * ((a.H / a.KH) / G);  // wavefronts per work item
-  (void)units;
+  const QuantPass pass = shared_ok ? quant_pass(B, units, a.max_pp, D) : QuantPass::kItems;
+  // (balanced: for the two passes enqueued apart, which leave partials)
+  const bool shared = shared_ok && pass != QuantPass::kItems;
   a.B = B;
   const long cap = items_capacity(B, a.KH);
   const size_t need = header_bytes(B) + (size_t)cap * a.H * (D + 2) * sizeof(float);
@@ -749,6 +780,20 @@ int run_decode(DecodeArgs a, int kind, float* out, void* workspace, size_t works
   a.part_acc = reinterpret_cast<float*>(static_cast<char*>(workspace) + header_bytes(B));
   a.part_ml = a.part_acc + (size_t)cap * a.H * D;
   a.qscale = scale * kLog2e;
+  if (shared_ok && pass == QuantPass::kBalanced && passes == kBoth) {
+    DecodeArgs ab = a;
+    ab.out = out;
+    const hipError_t e = launch_stream_balanced(ab, kind, B, D, G, st);
+    if (e == hipSuccess) {
+      clear_error();
+      return VRM_OK;
+    }
+    if (e != hipErrorInvalidValue) {
+      set_error("vrm_paged_decode: balanced kernel launch failed: %s", hipGetErrorString(e));
+      return (int)e;
+    }
+    // too much LDS for any launch shape: the shared rows below
+  }
   // with both passes in the call, the shared-items pass writes sequences of
   // one piece to out itself
   a.out = passes == kBoth && shared ? out : nullptr;
