@@ -134,34 +134,37 @@ def ptr(t) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
+_raw_stream = None  # torch's raw getter of a device's current stream
+
+
 def stream_of(t) -> int:
     """Raw handle of the current stream of t's device, the stream torch orders
     t's work on (torch's raw getter: the public Stream object costs about two
     microseconds per call)."""
-    import torch
+    global _raw_stream
+    if _raw_stream is None:
+        import torch
 
-    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-    if raw is not None:
-        return raw(t.get_device())
-    return torch.cuda.current_stream(t.device).cuda_stream
+        _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+            lambda index: torch.cuda.current_stream(index).cuda_stream)
+    return _raw_stream(t.get_device())
 
 
 def require_cuda(*tensors) -> None:
     """The kernels run on the GPU only; CPU tensors are an error, not a fallback."""
+    first = None
     for t in tensors:
-        if t is not None and not t.is_cuda:
+        if t is None:
+            continue
+        if not t.is_cuda:
             raise RuntimeError(
                 "vramancer_amd kernels run on the GPU; got a CPU tensor "
                 f"(shape {tuple(t.shape)}, dtype {t.dtype})"
             )
-    dev = None
-    for t in tensors:
-        if t is None:
-            continue
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise RuntimeError(f"tensors on different devices: {dev} and {t.device}")
+        if first is None:
+            first, index = t, t.get_device()
+        elif t.get_device() != index:
+            raise RuntimeError(f"tensors on different devices: {first.device} and {t.device}")
 
 
 _KV_CODES: dict = {}

@@ -46,6 +46,7 @@ from the small separate array: 1-7 % in the measured shapes).
 """
 from __future__ import annotations
 
+import functools
 from typing import Any, Optional, Tuple
 
 from . import _lib
@@ -78,6 +79,7 @@ def _codec_dtype(codec: str):
 LAYOUTS = ("inline", "plain")
 
 
+@functools.lru_cache(maxsize=256)
 def _inline_geometry(num_pages: int, num_kv_heads: int, page_size: int, head_dim: int, fp8: bool):
     """(slab bytes, byte offset of the scales, code strides, scale strides) of
     the inline layout; strides in elements of the code / float32 views.  The
@@ -127,7 +129,8 @@ def allocate_pool(num_pages: int, num_layers: int, num_kv_heads: int, head_dim: 
 
 
 def _same_strides(t, strides) -> bool:
-    return all(n <= 1 or st == want for n, st, want in zip(t.shape, t.stride(), strides))
+    got = t.stride()
+    return got == strides or all(n <= 1 or st == want for n, st, want in zip(t.shape, got, strides))
 
 
 def pool_layout(kv_pool, kv_scales) -> Optional[str]:

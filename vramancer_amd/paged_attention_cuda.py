@@ -22,8 +22,11 @@ extension.  Differences a caller can observe:
 """
 from __future__ import annotations
 
+import functools
 import math
 from typing import Any, Optional
+
+import torch
 
 from . import _lib
 
@@ -44,6 +47,14 @@ def has_cuda_paged_attention() -> bool:
     return _lib.available()
 
 
+@functools.lru_cache(maxsize=256)
+def _workspace_bytes(batch: int, num_heads: int, num_kv_heads: int, head_dim: int, max_pages_per_seq: int,
+                     page_size: int) -> int:
+    lib = _lib.load()
+    nsplit = lib.vrm_paged_decode_num_splits(batch, num_heads, num_kv_heads, max_pages_per_seq, page_size)
+    return max(lib.vrm_paged_decode_workspace_bytes(batch, num_heads, head_dim, max(nsplit, 1)), 16)
+
+
 def decode_workspace(batch: int, num_heads: int, num_kv_heads: int, head_dim: int, max_pages_per_seq: int,
                      device: Any, page_size: int = 16):
     """Allocates the split-K workspace a decode call of this shape needs.
@@ -51,12 +62,8 @@ def decode_workspace(batch: int, num_heads: int, num_kv_heads: int, head_dim: in
     Callers that decode in a loop can allocate it once and pass it as
     ``workspace=`` to avoid a per-call allocation.
     """
-    import torch
-
-    lib = _lib.load()
-    nsplit = lib.vrm_paged_decode_num_splits(batch, num_heads, num_kv_heads, max_pages_per_seq, page_size)
-    nbytes = lib.vrm_paged_decode_workspace_bytes(batch, num_heads, head_dim, max(nsplit, 1))
-    return torch.empty(max(nbytes, 16), dtype=torch.uint8, device=device)
+    nbytes = _workspace_bytes(batch, num_heads, num_kv_heads, head_dim, max_pages_per_seq, page_size)
+    return torch.empty(nbytes, dtype=torch.uint8, device=device)
 
 
 # The balanced decode (one workgroup per sequence and kv-head, partitions
@@ -71,8 +78,6 @@ def prefer_balanced(context_lens_host, num_kv_heads: int, kv_dtype) -> bool:
     """True when the balanced decode suits this batch: an int8 or fp8 pool, at
     least BALANCED_MIN_PAIRS (sequence, kv-head) pairs, and the longest context
     within BALANCED_MAX_SPREAD of the mean (host-side lengths, no device sync)."""
-    import torch
-
     if kv_dtype not in (torch.int8, torch.float8_e4m3fn):
         return False
     # built-in reductions over a list of ints (this runs once per layer call,
@@ -94,8 +99,6 @@ def check_outputs(query, out, workspace, page_table, context_lens) -> None:
     contiguous tensor, both on the query's device: the kernels write through
     their raw pointers.  ``page_table`` must be [B, max_pages] and
     ``context_lens`` [B] (the kernels read B rows of max_pages entries)."""
-    import torch
-
     B, H, D = query.shape
     if page_table.dim() != 2 or page_table.shape[0] != B or page_table.shape[1] < 1:
         raise RuntimeError(f"page_table must be [B={B}, max_pages >= 1], got {tuple(page_table.shape)}")
@@ -113,8 +116,6 @@ def check_outputs(query, out, workspace, page_table, context_lens) -> None:
 
 
 def _prepare(query, page_table, context_lens, scale):
-    import torch
-
     head_dim = query.shape[-1]
     if scale is None:
         scale = 1.0 / math.sqrt(head_dim)
@@ -150,8 +151,6 @@ def paged_attention_decode(
     selects the kernel (``prefer_balanced``): even batches over int8 / fp8
     pools take the balanced decode, which needs no workspace.
     """
-    import torch
-
     query, page_table, context_lens, scale = _prepare(query, page_table, context_lens, scale)
     _lib.require_cuda(query, kv_pool, page_table, context_lens, kv_scales)
     if kv_pool.dim() != 6:
@@ -216,8 +215,6 @@ def paged_attention_decode(
 
 
 def _check_lse(lse, B: int, H: int, device) -> None:
-    import torch
-
     if tuple(lse.shape) != (B, H) or lse.dtype != torch.float32 or not lse.is_contiguous() or lse.device != device:
         raise RuntimeError(f"lse must be a contiguous float32 [{B}, {H}] tensor on {device}")
 
@@ -226,8 +223,6 @@ def combine_attention(out1: Any, lse1: Any, out2: Any, lse2: Any, lse_out: Any =
     """Attention over the union of two disjoint token sets from the
     attentions over each ([..., D] float32 outputs with their [...] log-sum-exp
     of the scaled scores); rows where both sets are empty give zeros."""
-    import torch
-
     _lib.require_cuda(out1, lse1, out2, lse2, lse_out)
     if out1.shape != out2.shape or lse1.shape != lse2.shape or tuple(out1.shape[:-1]) != tuple(lse1.shape):
         raise RuntimeError("combine_attention: mismatched shapes")
@@ -260,8 +255,6 @@ def paged_attention_decode_q4(
     """Paged decode over the reference's asymmetric 4-bit pool
     (core/paged_attention_cuda.py:238-288): value = (nibble - zero) * scale with
     groups of 32 along head_dim, low nibble = even index."""
-    import torch
-
     query, page_table, context_lens, scale = _prepare(query, page_table, context_lens, scale)
     _lib.require_cuda(query, kv_pool_q4, kv_scales, kv_zeros, page_table, context_lens, out, workspace)
     check_outputs(query, out, workspace, page_table, context_lens)
