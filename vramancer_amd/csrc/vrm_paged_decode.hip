@@ -722,13 +722,16 @@ int check_kind_shape(int kind, int D, int PS, const char* who) {
 // to 64 tokens 86.7 -> 10.2 us, 8 of up to 2048 26.5 -> 17.9, 64 of up to 4096
 // 75.7 -> 69.0); where a batch loses, it loses at most 6 %.
 enum class QuantPass { kBalanced, kItems, kShared };
-QuantPass quant_pass(int B, int units, int max_pp, int D) {
+// The fits are of workgroups of 12 wavefronts: wide head groups, whose merge
+// area holds fewer in 64 KB, are left to the other two.
+QuantPass quant_pass(int B, int units, int max_pp, int G, int D) {
+  const bool full = balanced_lds_bytes(max_pp, kMaxBalancedWaves, G, D) <= kMaxBalancedLds;
   const double wgs = (double)B * units, work = wgs * max_pp;
   const double page = 0.018 + 0.00049 * D;
   const double balanced = 9.3 + (wgs <= 256 ? page * max_pp : 2 * page * max_pp * (wgs > 512 ? wgs / 512 : 1.0));
   const double items = 13.0 + 0.00052 * work * (D / 128.0);
   const double slack = B == 1 ? 1.0 : D >= 96 ? 2.5 : 1.5;
-  if (max_pp <= (wgs <= 512 ? 256 : 128) && balanced <= items + slack) return QuantPass::kBalanced;
+  if (full && max_pp <= (wgs <= 512 ? 256 : 128) && balanced <= items + slack) return QuantPass::kBalanced;
   if (work <= 4096 && (B > 1 || D >= 96)) return QuantPass::kItems;
   return QuantPass::kShared;
 }
