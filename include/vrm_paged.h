@@ -585,6 +585,23 @@ int vrm_paged_decode_tq_lse(const float* query, const uint8_t* tq_pool, const in
                             const float* signs, const float* jl, const float* angle_lut,
                             int with_qjl, vrm_stream_t stream);
 
+/*
+ * One decode step over a sequence set's TurboQuant pages and its uncompressed
+ * residual pages (a float pool [res_pages][1][2][KH][PS][D]; tq_pool holds one
+ * layer): the attention over the union, scores against the decompressed keys
+ * (no QJL term), as vrm_paged_decode_tq_lse, vrm_paged_decode_lse and
+ * vrm_attn_combine give it, with one merge of both passes' partials.  out
+ * [B][H][D] in out_dtype (VRM_SRC_F32 / _F16 / _BF16, rounded to nearest even).
+ * The two workspaces are distinct, each of vrm_paged_decode_workspace_bytes.
+ */
+int vrm_paged_decode_tq_residual(
+    const float* query, const uint8_t* tq_pool, const int32_t* tq_table, const int32_t* tq_lens,
+    int tq_pages, int tq_max_pp, const void* res_pool, int res_dtype, const int32_t* res_table,
+    const int32_t* res_lens, int res_pages, int res_max_pp, void* out, int out_dtype,
+    void* tq_workspace, size_t tq_workspace_bytes, void* res_workspace, size_t res_workspace_bytes,
+    int B, int H, int KH, int D, int PS, float scale, int bits, int qjl_dim, const float* signs,
+    const float* jl, const float* angle_lut, vrm_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -219,6 +219,16 @@ def test_manager_and_attend_entries_reject_bad_arguments(lib):
     assert lib.vrm_paged_decode_tq_lse(1, 1, 1, 1, 1, None, 1, 1 << 30, 2, 8, 8, 128, 16, 1, 4, 4, 0, 0.1, 3, 64,
                                        1, 1, 1, 0, None) == -1
 
+    def residual(res_dtype=_lib.VRM_KV_F32, out_dtype=_lib.VRM_SRC_BF16, tq_ws=1, res_ws=2, ws_bytes=1 << 30, H=8):
+        return lib.vrm_paged_decode_tq_residual(1, 1, 1, 1, 4, 4, 1, res_dtype, 1, 1, 4, 4, 1, out_dtype, tq_ws,
+                                                ws_bytes, res_ws, ws_bytes, 2, H, 8, 128, 16, 0.1, 3, 64, 1, 1, 1, None)
+
+    assert residual(res_dtype=_lib.VRM_KV_I8) == -1   # the residual is a float pool
+    assert residual(out_dtype=3) == -1
+    assert residual(res_ws=1) == -1                   # one workspace for both passes
+    assert residual(H=7) == -1
+    assert residual(ws_bytes=64) == -3
+
 
 def test_tq_slice_sizes():
     """Slice sizes of the two TurboQuant page layouts, from their field

@@ -104,3 +104,46 @@ def test_turboquant_cache_decode_attention_matches_materialised(setting):
         want = (w[..., None] * Vr).sum(2)
         err = (got - want).abs()
         assert (err <= 2e-3 + 1e-2 * want.abs()).all(), f"step {s}: max err {err.max():.3e} view {layer._view}"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("head_dim,bits,B,n_c,n_r", [
+    (64, 4, 4, 2000, 101),   # many partials of the pages, several of the residual
+    (64, 4, 1, 16, 1),       # one partial of each
+    (128, 3, 3, 160, 160),   # as many pages in both passes: their workspaces stay apart
+    (96, 2, 2, 3000, 33),
+    (256, 5, 2, 48, 17),     # head_dim above 128, generic pages
+])
+def test_merged_step_matches_two_decodes(dtype, head_dim, bits, B, n_c, n_r):
+    """The one merge of both passes' partials against the two decodes combined
+    by log-sum-exp.  The passes are the same, so float32 outputs differ by the
+    order of the sum over at most 600 partials of weight sum 1 (600 x 2^-24 of
+    the largest value) and by the rounding of the two log-sum-exps (|lse| < 16:
+    2^-20 of a value each), together below 4e-5 for |v| < 1 here; the 16-bit
+    outputs by one more rounding of theirs (2^-11, 2^-8 relative)."""
+    from vramancer_amd import tq_pages
+    from vramancer_amd.paged_attention_cuda import combine_attention, paged_attention_decode
+
+    _say(f"merged step {dtype} d{head_dim} b{bits} B{B} {n_c}+{n_r}")
+    torch.manual_seed(5)
+    cache = TurboQuantCache(1, head_dim, bits_per_angle=bits, residual_length=n_r, device=DEV, paged_attention=True)
+    layer = cache.layers[0]
+    g = torch.Generator().manual_seed(6)
+    for s in (n_c, n_r):
+        k = torch.randn(B, 2, s, head_dim, generator=g).to(DEV, dtype)
+        layer.update(k, (torch.rand(B, 2, s, head_dim, generator=g) - 0.5).to(DEV, dtype))
+    assert layer._view == (n_c, n_r)
+    q = torch.randn(B, 6, 1, head_dim, generator=g).to(DEV, dtype)
+    got = layer.attend_decode(q, 0.09)
+    assert got.dtype == dtype and tuple(got.shape) == (B, 1, 6, head_dim)
+    pj, pr = -(-n_c // 16), -(-n_r // 16)
+    q3 = q[:, :, 0].float().contiguous()
+    l1, l2 = (torch.empty((B, 6), device=DEV) for _ in range(2))
+    o1 = tq_pages.paged_attention_decode_turbo(q3, layer._tq_pool, layer._table("tq", pj), layer._lengths(n_c), 0,
+                                               layer.compressor, scale=0.09, lse=l1, qjl=False)
+    o2 = paged_attention_decode(q3, layer._res_pool, layer._table("res", pr), layer._lengths(n_r), 0, scale=0.09,
+                                lse=l2)
+    want = combine_attention(o1, l1, o2, l2)
+    rel = {torch.float32: 0.0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+    err = (got[:, 0].float() - want).abs()
+    assert (err <= 4e-5 + rel * want.abs()).all(), f"max err {err.max():.3e}"

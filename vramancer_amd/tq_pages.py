@@ -39,6 +39,7 @@ __all__ = [
     "quantize_pages",
     "read_pages",
     "paged_attention_decode_turbo",
+    "paged_attention_decode_residual",
 ]
 
 PAGE_SIZE = 16  # default tokens per page (the reference's)
@@ -257,4 +258,45 @@ def paged_attention_decode_turbo(query, tq_pool, page_table, context_lens, layer
             1 if qjl else 0, _lib.stream_of(query),
         )
     _lib.check(rc, "paged_attention_decode_turbo")
+    return out
+
+
+def paged_attention_decode_residual(query, tq_pool, tq_table, tq_lens, compressor, res_pool, res_table, res_lens,
+                                    scale: float, tq_workspace, res_workspace, out_dtype, page_size: int = PAGE_SIZE):
+    """[B, H, head_dim] attention over the union of one layer's TurboQuant
+    pages (scores against the decompressed keys) and its uncompressed residual
+    pages ([P, 1, 2, KH, page_size, head_dim], float), as the two decodes and
+    ``combine_attention`` give it, from one merge of both passes' partials.
+    query float32; the result is out_dtype where that is float32, float16 or
+    bfloat16, else float32."""
+    import torch
+
+    _check_compressor(compressor)
+    _lib.require_cuda(query, tq_pool, tq_table, tq_lens, res_pool, res_table, res_lens, tq_workspace, res_workspace)
+    P, L, KH = _pool_dims(tq_pool, compressor, page_size)
+    B, H, D = query.shape
+    if L != 1 or D != compressor.head_dim or H % KH or query.dtype != torch.float32 or not query.is_contiguous():
+        raise RuntimeError(f"query {query.dtype} {tuple(query.shape)} does not match the compressor's head_dim "
+                           f"{compressor.head_dim}, {KH} kv-heads and one layer")
+    if tuple(res_pool.shape[1:]) != (1, 2, KH, page_size, D) or not res_pool.is_contiguous():
+        raise RuntimeError(f"residual pool must be a contiguous [P, 1, 2, {KH}, {page_size}, {D}], got "
+                           f"{tuple(res_pool.shape)}")
+    for table, lens, ws in ((tq_table, tq_lens, tq_workspace), (res_table, res_lens, res_workspace)):
+        check_outputs(query, None, ws, table, lens)
+        if table.dtype != torch.int32 or lens.dtype != torch.int32 or not (table.is_contiguous() and
+                                                                           lens.is_contiguous()):
+            raise RuntimeError("page tables and lengths must be contiguous int32 tensors")
+    if out_dtype not in (torch.float32, torch.float16, torch.bfloat16):
+        out_dtype = torch.float32
+    out = torch.empty((B, H, D), dtype=out_dtype, device=query.device)
+    signs, jl, lut = _buffers(compressor, query.device)
+    rc = _lib.load().vrm_paged_decode_tq_residual(
+        _lib.ptr(query), _lib.ptr(tq_pool), _lib.ptr(tq_table), _lib.ptr(tq_lens), P, tq_table.shape[1],
+        _lib.ptr(res_pool), _lib.kv_dtype_code(res_pool.dtype), _lib.ptr(res_table), _lib.ptr(res_lens),
+        res_pool.shape[0], res_table.shape[1], _lib.ptr(out), _lib.src_dtype_code(out_dtype), _lib.ptr(tq_workspace),
+        tq_workspace.numel() * tq_workspace.element_size(), _lib.ptr(res_workspace),
+        res_workspace.numel() * res_workspace.element_size(), B, H, KH, D, page_size, float(scale),
+        compressor.bits_per_angle, compressor.qjl_dim, _lib.ptr(signs), _lib.ptr(jl), _lib.ptr(lut),
+        _lib.stream_of(query))
+    _lib.check(rc, "paged_attention_decode_residual")
     return out

@@ -49,7 +49,7 @@ from transformers.cache_utils import Cache, CacheLayerMixin
 
 from . import _lib, tq_pages
 from .kv_quantizer import KVCacheCompressor
-from .paged_attention_cuda import combine_attention, decode_workspace, paged_attention_decode
+from .paged_attention_cuda import decode_workspace, paged_attention_decode
 from .turboquant_cuda import CUDATurboQuantOps
 
 __all__ = ["TurboQuantLayer", "TurboQuantCache", "enable_paged_attention", "turbo_paged_attention",
@@ -273,8 +273,8 @@ class TurboQuantLayer(CacheLayerMixin):
             self._len_last = (n, torch.full((self._B,), n, dtype=torch.int32, device=self.device))
         return self._len_last[1]
 
-    def _workspace(self, H: int, pages: int):
-        key = (H, pages)
+    def _workspace(self, kind: str, H: int, pages: int):
+        key = (kind, H, pages)  # one per pass: the merge of a step reads both
         ws = self._ws.get(key)
         if ws is None:
             ws = decode_workspace(self._B, H, self._KH, self._D, pages, self.device)
@@ -285,33 +285,27 @@ class TurboQuantLayer(CacheLayerMixin):
         """One decode token per sequence, query [B, H, 1, D] -> [B, 1, H, D]:
         paged TurboQuant decode over the compressed tokens (scores against the
         decompressed keys, as the reference's cache hands them to attention:
-        no QJL term) and paged float decode over the residual, merged by
-        log-sum-exp."""
+        no QJL term) and paged float decode over the residual, whose partials
+        one kernel merges."""
         B, H, _, D = query.shape
         q = query[:, :, 0, :].float().contiguous()
         n_c, n_r = self._view
-        results = []
-        if n_c:
-            pj = -(-n_c // PAGE)
-            ctx = self._lengths(n_c)
-            lse = torch.empty((B, H), dtype=torch.float32, device=self.device)
-            out = tq_pages.paged_attention_decode_turbo(q, self._tq_pool, self._table("tq", pj), ctx, 0,
-                                                        self.compressor, scale=scale,
-                                                        workspace=self._workspace(H, pj), lse=lse, qjl=False)
-            results.append((out, lse))
-        if n_r:
-            pr = -(-n_r // PAGE)
-            ctx = self._lengths(n_r)
-            lse = torch.empty((B, H), dtype=torch.float32, device=self.device)
-            out = paged_attention_decode(q, self._res_pool, self._table("res", pr), ctx, 0, scale=scale,
-                                         workspace=self._workspace(H, pr), lse=lse)
-            results.append((out, lse))
-        if not results:
-            out = torch.zeros((B, H, D), dtype=torch.float32, device=self.device)
-        elif len(results) == 1:
-            out = results[0][0]
+        pj, pr = -(-n_c // PAGE), -(-n_r // PAGE)
+        if n_c and n_r:
+            out = tq_pages.paged_attention_decode_residual(
+                q, self._tq_pool, self._table("tq", pj), self._lengths(n_c), self.compressor, self._res_pool,
+                self._table("res", pr), self._lengths(n_r), scale, self._workspace("tq", H, pj),
+                self._workspace("res", H, pr), query.dtype)
+        elif n_c:
+            out = tq_pages.paged_attention_decode_turbo(
+                q, self._tq_pool, self._table("tq", pj), self._lengths(n_c), 0, self.compressor, scale=scale,
+                workspace=self._workspace("tq", H, pj),
+                lse=torch.empty((B, H), dtype=torch.float32, device=self.device), qjl=False)
+        elif n_r:
+            out = paged_attention_decode(q, self._res_pool, self._table("res", pr), self._lengths(n_r), 0,
+                                         scale=scale, workspace=self._workspace("res", H, pr))
         else:
-            out = combine_attention(results[0][0], results[0][1], results[1][0], results[1][1])
+            out = torch.zeros((B, H, D), dtype=torch.float32, device=self.device)
         return out.to(query.dtype).unsqueeze(1)
 
     # -- bookkeeping (core/turboquant_cache.py:256-299) ----------------------
