@@ -225,3 +225,29 @@ def test_decode_turbo_full_size_sampled_parity(name):
         ref = PD.paged_attention_decode_turbo(_params(comp), q[b:b + 1].cpu(), codes,
                                               torch.arange(n, dtype=torch.int32)[None], lens[b:b + 1].cpu())
         _assert_close(out[b:b + 1], ref, f"{name} seq {b}")
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4])
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("KH", [2, 3, 4])
+def test_lookup_tables_of_every_workgroup_size(bits, head_dim, KH):
+    """Workgroups of KH wavefronts fill the angle tables by whole planes or
+    entry by entry, whichever their size allows: a kv-head decoded among KH
+    gives the bits it gives alone (one partition of 4 pages either way)."""
+    _say(f"tables bits={bits} D={head_dim} KH={KH}")
+    torch.manual_seed(7)
+    comp = KVCacheCompressor(head_dim, bits).to(DEV)
+    k, v = (_student_t((4, KH, 16, head_dim), s).to(DEV) for s in (3, 4))
+    q = torch.randn(1, 2 * KH, head_dim, generator=torch.Generator().manual_seed(5)).to(DEV)
+    ids = torch.arange(4, dtype=torch.int32, device=DEV)
+    lens = torch.tensor([61], dtype=torch.int32, device=DEV)
+
+    def decode(heads):
+        pool = tq_pages.allocate_pool(4, 1, len(heads), comp, DEV)
+        tq_pages.quantize_pages(pool, 0, ids, k[:, heads].contiguous(), v[:, heads].contiguous(), comp)
+        rows = [2 * h + i for h in heads for i in (0, 1)]
+        return tq_pages.paged_attention_decode_turbo(q[:, rows], pool, ids[None], lens, 0, comp)
+
+    together = decode(list(range(KH)))
+    for h in range(KH):
+        assert torch.equal(together[:, 2 * h:2 * h + 2], decode([h])), h
