@@ -151,6 +151,17 @@ int vrm_paged_decode(const float* query, const void* kv_pool, const float* kv_sc
                      int B, int H, int KH, int D, int PS, int L, int P, int max_pp,
                      int layer_idx, float scale, int kv_dtype, vrm_stream_t stream);
 
+/* The partition pass that vrm_paged_decode takes for such a call, by its sizes
+ * alone: work items and a merge, rows of equal page counts and a merge, or one
+ * launch of a workgroup per sequence and one or two kv-heads (SPLIT: two for
+ * sequences far above the batch's mean).  Float and 4-bit pools always take
+ * work items.  Touches no stream; VRM_ERR_ARG for sizes no call can have. */
+#define VRM_PASS_ITEMS 0
+#define VRM_PASS_SHARED 1
+#define VRM_PASS_BALANCED 2
+#define VRM_PASS_BALANCED_SPLIT 3
+int vrm_paged_decode_pass(int B, int H, int KH, int D, int PS, int max_pp, int kv_dtype);
+
 /*
  * vrm_paged_decode without a workspace argument, for callers that cannot
  * allocate device memory (code under HIP graph capture, serving loops and

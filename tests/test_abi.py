@@ -337,3 +337,34 @@ def test_balanced_entry_rejects_bad_arguments(lib):
     bad = list(largs)
     bad[9] = 256
     assert g(*bad) == -2 and b"head_dim" in lib.vrm_last_error()
+
+
+@pytest.mark.parametrize("heads,B,max_pp,want", [
+    ((40, 8, 128), 64, 256, "split"),     # one round of two-unit workgroups: as fast as one can be if even
+    ((40, 8, 128), 64, 257, "split"),     # no cliff at the lengths that are timed most
+    ((40, 8, 128), 64, 300, "split"),
+    ((40, 8, 128), 64, 301, "shared"),    # one full sequence among short ones would set the time
+    ((40, 8, 128), 65, 100, "items"),     # 520 workgroups of a round of 512: two rounds, 60 us against 53
+    ((40, 8, 128), 65, 32, "balanced"),
+    ((40, 8, 128), 96, 100, "balanced"),  # the second round half full
+    ((40, 8, 128), 256, 100, "items"),    # skewed 86 us against 41
+    ((40, 8, 128), 33, 256, "items"),     # half of the CUs idle and the longest sequence sets the time
+    ((40, 8, 128), 8, 137, "items"),      # not the shared rows, which the cost says nothing about
+    ((40, 8, 128), 128, 512, "shared"),
+    ((12, 12, 64), 43, 100, "items"),
+    ((12, 12, 64), 21, 128, "balanced"),
+])
+def test_pass_of_int8_batches(lib, heads, B, max_pp, want):
+    """The pass is chosen from the sizes alone; the lines lie where no
+    distribution of lengths makes the choice much slower than the others."""
+    H, KH, D = heads
+    names = {0: "items", 1: "shared", 2: "balanced", 3: "split"}
+    for code in (3, 4):  # int8, fp8
+        assert names[lib.vrm_paged_decode_pass(B, H, KH, D, 16, max_pp, code)] == want
+
+
+def test_pass_of_other_calls(lib):
+    f = lib.vrm_paged_decode_pass
+    assert f(8, 40, 8, 128, 16, 64, 2) == 0  # float pools
+    assert f(8, 40, 8, 256, 16, 64, 3) == 0 and f(8, 40, 8, 128, 32, 64, 3) == 0  # other shapes
+    assert f(8, 40, 7, 128, 16, 64, 3) == -1 and f(0, 40, 8, 128, 16, 64, 3) == -1 and f(8, 40, 8, 128, 16, 64, 9) == -1

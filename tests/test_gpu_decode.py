@@ -797,6 +797,38 @@ def test_inline_layout_decodes_like_the_plain_layout(dtype, D, PS):
     _assert_close(outs["inline"][0], PD.paged_attention_decode(q, pool, table, lens, 1, kv_scales=sc), "oracle")
 
 
+@pytest.mark.parametrize("dtype", [torch.int8, torch.float8_e4m3fn], ids=["int8", "fp8"])
+@pytest.mark.parametrize("B,H,KH,D,pin", [(64, 40, 8, 128, [(3, 2071)]), (64, 8, 8, 64, [(0, 2900), (63, 2833)]),
+                                          (58, 5, 5, 96, [(57, 1640)])],
+                         ids=["D128", "two-long", "odd-units"])
+def test_long_sequences_among_short_ones_take_two_workgroups(dtype, B, H, KH, D, pin):
+    """A batch of 257 to 512 (sequence, kv-head) pairs under a table of more
+    than 100 pages: sequences of 96 pages and three times the mean are streamed
+    by a workgroup per kv-head (the last of an odd number of kv-heads has no
+    partner), the others by one per two; absent pages, empty sequences and the
+    log-sum-exp as elsewhere."""
+    _say(f"split {dtype} B{B} KH{KH} D{D}")
+    ctxs = [(37 * i) % 290 for i in range(B)]  # 0 .. 18 pages
+    for b, n in pin:
+        ctxs[b] = n
+    q, pool, sc, table, lens = _pool_case(dtype, B, H, KH, D, ctxs, seed=B + D)
+    width = table.shape[1]
+    code = _lib.VRM_KV_I8 if dtype == torch.int8 else _lib.VRM_KV_FP8E4M3
+    assert _lib.load().vrm_paged_decode_pass(B, H, KH, D, 16, width, code) == 3
+    want = PD.paged_attention_decode(q, pool, table, lens, 1, kv_scales=sc)
+    d = [t.to(DEV) for t in (q, pool, sc, table, lens)]
+    out = paged_attention_decode(d[0], d[1], d[3], d[4], 1, kv_scales=d[2])
+    torch.cuda.synchronize()
+    _assert_close(out, want, "split")
+    # an absent page (the oracle has none): against the workgroups of two units
+    d[3][pin[0][0], 5] = -1
+    lse, lse_bal = torch.empty(B, H, device=DEV), torch.empty(B, H, device=DEV)
+    out = paged_attention_decode(d[0], d[1], d[3], d[4], 1, kv_scales=d[2], lse=lse)
+    torch.cuda.synchronize()
+    _assert_rerun(out, _balanced(*d, 1, lse=lse_bal), True, "split with an absent page")
+    _assert_rerun(lse, lse_bal, True, "lse of the split")
+
+
 def test_balanced_decode_refuses_d256_and_the_api_falls_back():
     """D = 256 is outside the balanced decode (VRM_ERR_UNSUPPORTED); the
     Python API then runs the work-item decode for the same even batch."""

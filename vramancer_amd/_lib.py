@@ -45,6 +45,7 @@ SIGNATURES = {
     "vrm_abi_version": (_i, []),
     "vrm_last_error": (ctypes.c_char_p, []),
     "vrm_kv_slab_bytes": (_sz, [_i, _i, _i, _i]),
+    "vrm_paged_decode_pass": (_i, [_i] * 7),
     "vrm_paged_decode_num_splits": (_i, [_i, _i, _i, _i, _i]),
     "vrm_paged_decode_workspace_bytes": (_sz, [_i, _i, _i, _i]),
     "vrm_paged_decode": (_i, [_p, _p, _p, _p, _p, _p, _p, _sz] + [_i] * 9 + [_f, _i, _p]),

@@ -320,6 +320,7 @@ constexpr int kMaxUnitsPerWg = 4;  // page-pair counters the LDS layout leaves r
 constexpr int kIdBucketBits = 6;   // a work item's pages are read in 2^6 buckets of ascending page id
 constexpr int kIdBuckets = 1 << kIdBucketBits;
 constexpr size_t kMaxBalancedLds = 64 * 1024;
+constexpr int kSplitMinPages = 96;  // pages from which a sequence is worth two workgroups (split)
 // LDS one workgroup of the shared-items pass may take on the current device
 // (its 12-wavefront workgroups hold a CU each, so beyond 64 KB costs no
 // occupancy): the device's per-workgroup limit, at most 160 KB.
@@ -337,10 +338,12 @@ inline size_t balanced_lds_bytes(int max_pp, int W, int G, int D) {
 // no workspace, no merge launch.  Correct for any context lengths; its time follows the
 // longest sequence, so it suits batches of about equal lengths.  kind is
 // K_I8 or K_FP8, D a multiple of 16 from 64 to 128.
+// split: sequences far above the batch's mean take a workgroup per unit
+// (decided on the device), so that no other needs to be close to the longest.
 // loads_only: the measuring build that issues the same loads and computes
 // nothing (a checksum of the words goes to out).
 hipError_t launch_stream_balanced(const DecodeArgs& a, int kind, int B, int D, int G, hipStream_t st,
-                                  bool loads_only = false);
+                                  bool loads_only = false, bool split = false);
 
 // The shared-items partition pass: balanced workgroups of 12 wavefronts (2
 // units x 6, or 4 x 3 when the batch has more sequences than a resident round

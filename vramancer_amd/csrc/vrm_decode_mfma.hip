@@ -824,6 +824,19 @@ __device__ __forceinline__ DecodeArgs kernel_args_afresh() {
   return ai;
 }
 
+// True for a sequence that the batch would wait for: 96 pages or more, and
+// above twice the batch's mean (none in an even batch, none among lengths
+// spread evenly from an eighth of the longest up: with a lower line those
+// lose, 64 of up to 64 pages 21 -> 31 us at 4/3 of the mean).
+__device__ __forceinline__ bool split_sequence(const DecodeArgs& a, int b) {
+  const int lane = __lane_id();
+  int total = 0;
+  for (int c = 0; c < a.B; c += 64) total += c + lane < a.B ? seq_pages(a.ctx_lens[c + lane], a.max_pp) : 0;
+  total = wave_sum_int(total);
+  const int pages = seq_pages(a.ctx_lens[b], a.max_pp);
+  return pages >= kSplitMinPages && (long long)pages * a.B > 3LL * total;
+}
+
 // grid: (work item, unit group), balanced: (sequence, unit group).  ITEMS:
 // (unit group, row), one resident round (a.target rows), each workgroup
 // taking the pieces of its row (find_piece) in turn: every row carries the
@@ -831,9 +844,20 @@ __device__ __forceinline__ DecodeArgs kernel_args_afresh() {
 // ones.  Between two pieces every wavefront has passed the first piece's
 // merge barrier, so the next piece's page ids and counters overwrite nothing
 // still read.
-template <int KIND, int D, bool BALANCED, bool LOADS = false, bool ITEMS = false, int UPW = kUnitsPerWg>
+//
+// SPLIT (balanced): grid z = 2.  A sequence that the batch would wait for is
+// streamed by two workgroups, one unit each with all wavefronts on it, so that
+// a lone long sequence among short ones costs half its pages' time.  The
+// workgroups of z = 0 have nothing to do for the others and leave at once;
+// they go first, since workgroups dispatched behind the whole batch would
+// start late (one of 256 pages among 47 short ones 32 us, 42 with them last;
+// 64 of 256 pages each 96.5 us, 95.9 without them), and they take the
+// sequences five further on, or at B % 64 == 0 both would queue on one CU.
+template <int KIND, int D, bool BALANCED, bool LOADS = false, bool ITEMS = false, int UPW = kUnitsPerWg,
+          bool SPLIT = false>
 __global__ void __launch_bounds__(64 * (BALANCED ? kMaxBalancedWaves : kMaxWaves))
     decode_stream_kernel(DecodeArgs a, int G) {
+  static_assert(!SPLIT || (BALANCED && !LOADS && !ITEMS && UPW == 2), "two units to split");
   static_assert(UPW == kUnitsPerWg || (BALANCED && !LOADS && UPW <= kMaxUnitsPerWg && kMaxBalancedWaves % UPW == 0),
                 "only balanced builds that compute take other unit counts");
   if constexpr (ITEMS) {
@@ -841,6 +865,12 @@ __global__ void __launch_bounds__(64 * (BALANCED ? kMaxBalancedWaves : kMaxWaves
       const DecodeArgs ai = kernel_args_afresh();
       items = stream_item<KIND, D, BALANCED, LOADS, ITEMS, UPW>(ai, G, item, blockIdx.x);  // 0: no such piece
     }
+  } else if constexpr (SPLIT) {
+    const int b = blockIdx.z ? blockIdx.x : (blockIdx.x + 5) % a.B;
+    if (split_sequence(a, b))
+      stream_item<KIND, D, BALANCED, LOADS, ITEMS, 1>(a, G, b, 2 * blockIdx.y + blockIdx.z);
+    else if (blockIdx.z)
+      stream_item<KIND, D, BALANCED, LOADS, ITEMS, UPW>(a, G, b, blockIdx.y);
   } else {
     stream_item<KIND, D, BALANCED, LOADS, ITEMS, UPW>(a, G, blockIdx.x, blockIdx.y);
   }
@@ -1550,7 +1580,7 @@ hipError_t launch_d(const DecodeArgs& a, int B, int D, int G, hipStream_t st) {
 // and 64 KB of LDS.  Returns hipErrorInvalidValue when even WPU = 1 does not
 // fit (page tables too wide for the LDS copy of the ids).
 template <int KIND, int D, bool LOADS>
-hipError_t launch_balanced_d(const DecodeArgs& a, int B, int G, hipStream_t st) {
+hipError_t launch_balanced_d(const DecodeArgs& a, int B, int G, hipStream_t st, bool split) {
   const int units = a.KH * ((a.H / a.KH) / G);
   const int wgs_y = (units + kUnitsPerWg - 1) / kUnitsPerWg;
   // the launch shape of the decode itself, for both builds
@@ -1571,6 +1601,13 @@ hipError_t launch_balanced_d(const DecodeArgs& a, int B, int G, hipStream_t st) 
     const size_t lds = balanced_lds_bytes(a.max_pp, W, G, D);
     if (lds > kMaxBalancedLds) continue;
     if (wpu > 1 && (long)B * wgs_y * W > resident) continue;
+    if constexpr (!LOADS) {
+      if (split && wpu == 6) {
+        hipLaunchKernelGGL((decode_stream_kernel<KIND, D, true, false, false, 2, true>), dim3(B, wgs_y, 2),
+                           dim3(64 * W), lds, st, a, G);
+        return hipGetLastError();
+      }
+    }
     hipLaunchKernelGGL((decode_stream_kernel<KIND, D, true, LOADS>), dim3(B, wgs_y, 1), dim3(64 * W), lds, st, a,
                        G);
     return hipGetLastError();
@@ -1628,13 +1665,13 @@ hipError_t launch_shared_items_kind(const DecodeArgs& a, int B, int D, int G, hi
 }
 
 template <int KIND, bool LOADS>
-hipError_t launch_balanced_kind(const DecodeArgs& a, int B, int D, int G, hipStream_t st) {
+hipError_t launch_balanced_kind(const DecodeArgs& a, int B, int D, int G, hipStream_t st, bool split) {
   switch (D) {
-    case 64: return launch_balanced_d<KIND, 64, LOADS>(a, B, G, st);
-    case 80: return launch_balanced_d<KIND, 80, LOADS>(a, B, G, st);
-    case 96: return launch_balanced_d<KIND, 96, LOADS>(a, B, G, st);
-    case 112: return launch_balanced_d<KIND, 112, LOADS>(a, B, G, st);
-    case 128: return launch_balanced_d<KIND, 128, LOADS>(a, B, G, st);
+    case 64: return launch_balanced_d<KIND, 64, LOADS>(a, B, G, st, split);
+    case 80: return launch_balanced_d<KIND, 80, LOADS>(a, B, G, st, split);
+    case 96: return launch_balanced_d<KIND, 96, LOADS>(a, B, G, st, split);
+    case 112: return launch_balanced_d<KIND, 112, LOADS>(a, B, G, st, split);
+    case 128: return launch_balanced_d<KIND, 128, LOADS>(a, B, G, st, split);
     default: return hipErrorInvalidValue;
   }
 }
@@ -1650,15 +1687,15 @@ hipError_t launch_q4(const DecodeArgs& a, int B, int G, hipStream_t st) {
 }  // namespace
 
 hipError_t launch_stream_balanced(const DecodeArgs& a, int kind, int B, int D, int G, hipStream_t st,
-                                  bool loads_only) {
+                                  bool loads_only, bool split) {
   if (G < 1 || G > 16) return hipErrorInvalidValue;
   switch (kind) {
     case K_I8:
-      return loads_only ? launch_balanced_kind<K_I8, true>(a, B, D, G, st)
-                        : launch_balanced_kind<K_I8, false>(a, B, D, G, st);
+      return loads_only ? launch_balanced_kind<K_I8, true>(a, B, D, G, st, false)
+                        : launch_balanced_kind<K_I8, false>(a, B, D, G, st, split);
     case K_FP8:
-      return loads_only ? launch_balanced_kind<K_FP8, true>(a, B, D, G, st)
-                        : launch_balanced_kind<K_FP8, false>(a, B, D, G, st);
+      return loads_only ? launch_balanced_kind<K_FP8, true>(a, B, D, G, st, false)
+                        : launch_balanced_kind<K_FP8, false>(a, B, D, G, st, split);
     default: return hipErrorInvalidValue;
   }
 }

@@ -745,21 +745,40 @@ int check_kind_shape(int kind, int D, int PS, const char* who) {
 // from what the host knows: sequences, (kv-head, head chunk) units and the
 // page table's width, the longest a sequence can be.
 //   balanced: one workgroup per sequence and unit (or two), one launch, time
-//     by the longest sequence;
+//     by the longest sequence; with two units a workgroup, sequences far above
+//     the mean take two workgroups (split);
 //   items: 4 pages or more per wavefront and a merge launch, for few pages;
 //   shared: rows of equal page counts and a merge launch, for the rest.
-// The times are fits to 576 batches (1 to 128 sequences of 64 to 65,536
-// tokens, equal and drawn from an eighth of the longest up, 40 / 8 and 28 / 4
-// heads of 128 and 12 / 12 of 64): a workgroup's 9.3 us and 0.08 us per page of
-// 128 dims (all 12 wavefronts on one unit; twice that with two units, from 256
-// workgroups on), against 13 us and 0.52 ns per page and unit.  The slack of
-// 1 to 2.5 us, and 256 pages at most, keep a table that is wider than its
-// sequences from costing more than the shared rows would have.  Over those
-// batches the choice takes 0.63 of the shared rows' time (128 sequences of up
-// to 64 tokens 86.7 -> 10.2 us, 8 of up to 2048 26.5 -> 17.9, 64 of up to 4096
-// 75.7 -> 69.0); where a batch loses, it loses at most 6 %.
+// Measured over 12,038 batches: 40 / 8 and 28 / 4 heads of 128 and 12 / 12 of 64,
+// 1 to 512 sequences, tables of 2 to 320 pages (some of them four times the
+// longest sequence), equal lengths, uniform from an eighth of the longest up,
+// and skewed ones (one long sequence, or every eighth, among ones of up to 16
+// pages; one among ones of a thirtieth to a twelfth).  The lines lie where the
+// worst of these against the fastest pass is least:
+//   up to 256 workgroups balanced follows its cost below; past it, items to
+//     128 workgroups (at 8 sequences of up to 200 pages 0.76 of the shared
+//     rows or less), since the shared rows are the fastest for equal lengths
+//     that fill their rows evenly but two to thirteen times slower than the
+//     others for skewed ones;
+//   257 to 512, split above 100 pages: up to 300 pages where the cost favours
+//     it by more the longer the table (64 of 256 pages each 96 us against 99;
+//     one of them among short ones 32 us against 42, 51 without the split);
+//   above 512 the workgroups queue for the CUs: 65 sequences of 8 units take
+//     60 us at 100 pages each where 64 take 38 and items 53, so only up to 32
+//     pages, 128 if the last round of 512 is at least half full, 80 once there
+//     are three rounds; then items up to 128 pages, and the shared rows.
+// Over those batches the choice takes 0.59 of the shared rows' time.  Where it
+// loses to them, it is by at most 22 % (192 sequences of 32 pages under a table
+// of 128: 60 us against 49; 128 sequences, one of 128 pages and the others of
+// 10: 59 against 49).  To the fastest of the three balanced and items lose up
+// to 2.3 times, to skewed lengths that the host cannot see (64 sequences of 12
+// units, one of 128 pages: 37 us against 16), the shared rows, which take the
+// rest as they always did, up to 3.9 times.
+// The cost is a fit to equal and uniform batches: a workgroup's 9.3 us and
+// 0.08 us per page of 128 dims (all 12 wavefronts on one unit; twice that with
+// two units), against 13 us and 0.52 ns per page and unit of the items.
 enum class QuantPass { kBalanced, kItems, kShared };
-// The fits are of workgroups of 12 wavefronts: wide head groups, whose merge
+// All of this is of workgroups of 12 wavefronts: wide head groups, whose merge
 // area holds fewer in 64 KB, are left to the other two.
 QuantPass quant_pass(int B, int units, int max_pp, int G, int D) {
   const bool full = balanced_lds_bytes(max_pp, kMaxBalancedWaves, G, D) <= kMaxBalancedLds;
@@ -768,9 +787,34 @@ QuantPass quant_pass(int B, int units, int max_pp, int G, int D) {
   const double balanced = 9.3 + (wgs <= 256 ? page * max_pp : 2 * page * max_pp * (wgs > 512 ? wgs / 512 : 1.0));
   const double items = 13.0 + 0.00052 * work * (D / 128.0);
   const double slack = B == 1 ? 1.0 : D >= 96 ? 2.5 : 1.5;
-  if (full && max_pp <= (wgs <= 512 ? 256 : 128) && balanced <= items + slack) return QuantPass::kBalanced;
-  if (work <= 4096 && (B > 1 || D >= 96)) return QuantPass::kItems;
-  return QuantPass::kShared;
+  bool few = (work <= 4096 && (B > 1 || D >= 96)) || (D >= 96 && wgs <= 128 && max_pp <= 256);
+  bool fits;
+  if (wgs <= 256) {
+    fits = max_pp <= 256 && balanced <= items + slack;
+  } else if (wgs <= 512) {
+    few = max_pp <= 256;
+    if (max_pp <= 200)
+      fits = balanced <= items + slack;
+    else
+      fits = max_pp <= 300 && balanced <= items * (max_pp <= 256 ? 0.80 : 0.65) * (D >= 96 ? 1.0 : 1.11);
+  } else {
+    few = max_pp <= 128;
+    const bool half = ((long)B * units - 1) % 512 >= 255;
+    fits = max_pp <= (wgs > 1024 ? 80 : half ? 128 : 32) && balanced <= items + slack;
+  }
+  if (full && fits) return QuantPass::kBalanced;
+  return few ? QuantPass::kItems : QuantPass::kShared;
+}
+// Shapes the shared-items pass takes: page 16, head_dim 64 .. 128 and a page
+// table whose LDS copy fits.
+bool shared_items_ok(int kind, int max_pp, int G, int D, int PS) {
+  return (kind == K_I8 || kind == K_FP8) && PS == kPS && D >= 64 && D <= 128 && D % 16 == 0 &&
+         balanced_lds_bytes(max_pp, kMaxBalancedWaves, G, D) <= shared_items_max_lds();
+}
+// Below some 100 pages every batch is faster without the split.
+bool balanced_split(int B, int units, int max_pp) {
+  const long wgs = (long)B * units;
+  return wgs > 256 && wgs <= 512 && max_pp > 100;
 }
 
 int run_decode(DecodeArgs a, int kind, float* out, void* workspace, size_t workspace_bytes, int B, int D, int PS,
@@ -803,8 +847,7 @@ int run_decode(DecodeArgs a, int kind, float* out, void* workspace, size_t works
   // int8 / fp8 at page 16 and head_dim 64 .. 128: the work items' pages are
   // shared by balanced workgroups (12 wavefronts, page pairs handed out in
   // LDS), when the page table fits their LDS copy
-  const bool shared_ok = (kind == K_I8 || kind == K_FP8) && PS == kPS && D >= 64 && D <= 128 && D % 16 == 0 &&
-                         balanced_lds_bytes(a.max_pp, kMaxBalancedWaves, G, D) <= shared_items_max_lds();
+  const bool shared_ok = shared_items_ok(kind, a.max_pp, G, D, PS);
   const int units = a.KH * ((a.H / a.KH) / G);  // wavefronts per work item
   const QuantPass pass = shared_ok ? quant_pass(B, units, a.max_pp, G, D) : QuantPass::kItems;
   // (balanced: for the two passes enqueued apart, which leave partials)
@@ -823,7 +866,8 @@ int run_decode(DecodeArgs a, int kind, float* out, void* workspace, size_t works
   if (shared_ok && pass == QuantPass::kBalanced && passes == kBoth) {
     DecodeArgs ab = a;
     ab.out = out;
-    const hipError_t e = launch_stream_balanced(ab, kind, B, D, G, st);
+    const hipError_t e =
+        launch_stream_balanced(ab, kind, B, D, G, st, false, balanced_split(B, units, a.max_pp));
     if (e == hipSuccess) {
       clear_error();
       return VRM_OK;
@@ -1072,6 +1116,25 @@ extern "C" int vrm_paged_decode_num_splits(int B, int H, int KH, int max_pp, int
 extern "C" size_t vrm_paged_decode_workspace_bytes(int B, int H, int D, int nsplit) {
   if (B <= 0 || H <= 0 || D <= 0 || nsplit <= 0) return 0;
   return header_bytes(B) + (size_t)B * H * nsplit * (D + 2) * sizeof(float);
+}
+
+extern "C" int vrm_paged_decode_pass(int B, int H, int KH, int D, int PS, int max_pp, int kv_dtype) {
+  const int kind = kind_of(kv_dtype);
+  if (kind < 0 || B <= 0 || H <= 0 || KH <= 0 || D <= 0 || PS <= 0 || max_pp <= 0 || H % KH) {
+    set_error("vrm_paged_decode_pass: bad arguments (B=%d H=%d KH=%d D=%d PS=%d max_pp=%d kv_dtype=%d)", B, H, KH, D,
+              PS, max_pp, kv_dtype);
+    return VRM_ERR_ARG;
+  }
+  clear_error();
+  const int G = pick_group_tile(H / KH, 16);
+  if (!shared_items_ok(kind, max_pp, G, D, PS)) return VRM_PASS_ITEMS;
+  const int units = KH * ((H / KH) / G);
+  switch (quant_pass(B, units, max_pp, G, D)) {
+    case QuantPass::kBalanced:
+      return balanced_split(B, units, max_pp) ? VRM_PASS_BALANCED_SPLIT : VRM_PASS_BALANCED;
+    case QuantPass::kItems: return VRM_PASS_ITEMS;
+    default: return VRM_PASS_SHARED;
+  }
 }
 
 extern "C" int vrm_paged_decode(const float* query, const void* kv_pool, const float* kv_scales,
