@@ -84,6 +84,76 @@ extern "C" long fast_bin_mismatches(int bits, int level0, long n, uint64_t seed,
     default: return bins<4, true>(n, seed, edges);
   }
 }
+// Multiples of pi / 4, by operands of one magnitude and by signed zeros: bins
+// that differ from the defining atan2, or that are left to it.
+template <int BITS, bool L0> static long symmetric() {
+  const float lo0 = (float)-3.141592653589793, r0 = (float)6.283185307179586, r1 = (float)1.5707963267948966;
+  const float mags[] = {1e-37f, 3e-20f,  // normal: the reciprocal of a denormal overflows, which is an edge
+                         1e-6f, 0.3f, 1.f, 2.7182817f, 5e4f, 1e15f};
+  long bad = 0;
+  for (float m : mags) {
+    if (!L0 && m < 1e-6f) continue;  // radii carry a floor of 1e-6
+    for (int c = 0; c < 32; ++c) {
+      float x = c & 4 ? 0.f : m, y = c & 8 ? 0.f : m;
+      if (c & 16) x *= 0.5f, y *= 0.5f;
+      x = c & 1 ? -x : x;
+      y = c & 2 ? -y : y;
+      if (!L0) { x = m; y = m; }
+      bool edge;
+      const int got = vrm_tq_bin::fast_bin<BITS, L0>(x, y, 1.0f / fmaxf(fabsf(x), fabsf(y)), edge);
+      const float th = vrm_fdlibm::atan2f(y, x);
+      const float d = th - lo0;
+      const float nrm = L0 ? d / r0 : th / r1;
+      const float t = nrm * (float)(1 << BITS);
+      int ref = (int)t;
+      ref = ref < 0 ? 0 : ref > (1 << BITS) - 1 ? (1 << BITS) - 1 : ref;
+      if (edge || got != ref) ++bad;
+    }
+  }
+  return bad;
+}
+// The ends of the range above level 0: small angles to x and to y.
+template <int BITS> static long ends(long n) {
+  uint64_t s = 88172645463325252ull;
+  auto next = [&]() { s ^= s << 13; s ^= s >> 7; s ^= s << 17; return s; };
+  long bad = 0;
+  for (long i = 0; i < n; ++i) {
+    float x = ldexpf(1.0f + (float)(next() & 0x7fffff) / 8388608.0f, (int)(next() % 20));
+    float y = x * ldexpf(1.0f + (float)(next() & 0x7fffff) / 8388608.0f, -20 - (int)(next() % 16));
+    if (i & 1) { const float z = x; x = y; y = z; }
+    bool edge;
+    const int got = vrm_tq_bin::fast_bin<BITS, false>(x, y, 1.0f / fmaxf(x, y), edge);
+    const float nrm = vrm_fdlibm::atan2f(y, x) / (float)1.5707963267948966;
+    const float t = nrm * (float)(1 << BITS);
+    int ref = (int)t;
+    ref = ref > (1 << BITS) - 1 ? (1 << BITS) - 1 : ref;
+    if (edge || got != ref) ++bad;
+  }
+  return bad;
+}
+extern "C" long end_mismatches(long n) { return ends<2>(n) + ends<3>(n) + ends<4>(n); }
+// Above level 0, pi / 4 within 64 ulp: the same.
+template <int BITS> static long middle(long n) {
+  uint64_t s = 88172645463325252ull;
+  auto next = [&]() { s ^= s << 13; s ^= s >> 7; s ^= s << 17; return s; };
+  long bad = 0;
+  for (long i = 0; i < n; ++i) {
+    const float x = ldexpf(1.0f + (float)(next() & 0x7fffff) / 8388608.0f, (int)(next() % 60) - 19);
+    const float y = vrm_fdlibm::bitsf(vrm_fdlibm::fbits(x) + (uint32_t)(next() % 129) - 64u);
+    bool edge;
+    const int got = vrm_tq_bin::fast_bin<BITS, false>(x, y, 1.0f / fmaxf(x, y), edge);
+    const float nrm = vrm_fdlibm::atan2f(y, x) / (float)1.5707963267948966;
+    const float t = nrm * (float)(1 << BITS);
+    if (edge || got != (int)t) ++bad;
+  }
+  return bad;
+}
+extern "C" long middle_mismatches(long n) { return middle<2>(n) + middle<3>(n) + middle<4>(n); }
+extern "C" long symmetric_mismatches() {
+  return symmetric<2, false>() + symmetric<2, true>() + symmetric<3, false>() + symmetric<3, true>() +
+         symmetric<4, false>() + symmetric<4, true>();
+}
+extern "C" uint32_t div_sqrt128_bits(float x) { return vrm_fdlibm::fbits(vrm_tq_bin::div_sqrt128(x)); }
 extern "C" long div_sqrt128_mismatches(int exponent) {
   const volatile float root = (float)sqrt(128.0);
   long bad = 0;
@@ -150,6 +220,29 @@ def test_fast_bin_is_the_defined_bin_off_the_edges(hostlib, bits, level0):
     assert hostlib.fast_bin_mismatches(bits, level0, n, 7 + bits, ctypes.byref(edges)) == 0
     # the ordinary quarter of the draws is hardly ever at an edge
     assert edges.value < 0.76 * n
+
+
+def test_fast_bin_knows_the_multiples_of_a_quarter_pi(hostlib):
+    hostlib.symmetric_mismatches.restype = ctypes.c_long
+    assert hostlib.symmetric_mismatches() == 0
+
+
+def test_fast_bin_decides_the_middle_of_the_range(hostlib):
+    hostlib.middle_mismatches.restype = ctypes.c_long
+    hostlib.middle_mismatches.argtypes = [ctypes.c_long]
+    assert hostlib.middle_mismatches(3_000_000) == 0
+
+
+def test_fast_bin_has_no_edge_at_the_ends_of_the_range(hostlib):
+    hostlib.end_mismatches.restype = ctypes.c_long
+    hostlib.end_mismatches.argtypes = [ctypes.c_long]
+    assert hostlib.end_mismatches(2_000_000) == 0
+
+
+def test_div_sqrt128_keeps_the_sign_of_zero(hostlib):
+    hostlib.div_sqrt128_bits.restype = ctypes.c_uint32
+    hostlib.div_sqrt128_bits.argtypes = [ctypes.c_float]
+    assert hostlib.div_sqrt128_bits(0.0) == 0 and hostlib.div_sqrt128_bits(-0.0) == 0x80000000
 
 
 @pytest.mark.parametrize("exponent", [-100, -3, 0, 1, 100])
