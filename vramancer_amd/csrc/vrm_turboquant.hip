@@ -62,11 +62,12 @@ constexpr int kBulkMinRows = 4096;
 // size (2 x 8 rows 7.1 / 6.4 us, 2 x 4096 16.7 / 8.1).
 constexpr int kTileMinRows = 2048;
 constexpr int kTileMaxRows = 0x7fffff00;
-// Rows from which raw codes at padded dim 128 are decompressed 16 rows per
-// wavefront (row kernel / tiles at 3 bits: 4096 rows 4.3 / 5.3 us, 16,384 7.5 /
-// 6.1, 65,536 23.4 / 16.4; padded dim 64 is as fast or faster tiled from one
-// row on, 65,536 rows 14.1 / 7.2).
+// Rows from which raw codes are decompressed 16 rows per wavefront (row kernel /
+// tiles at 3 bits: padded dim 128 4096 rows 4.3 / 5.3 us, 16,384 7.5 / 6.1,
+// 65,536 23.4 / 16.4; padded dim 64 512 rows 3.6 / 4.4, 8192 4.5 / 4.7, 12,000
+// 5.2 / 4.7, 65,536 15.4 / 8.3).
 constexpr int kTileMinDecompressRows = 16384;
+constexpr int kTileMinDecompressRows64 = 10240;
 
 // LUT_LDS: the angle table (4 x 2^bits floats, bits <= 4) is read from LDS.
 template <int SRC, int PD, int ROWS, bool LUT_LDS>
@@ -712,7 +713,7 @@ extern "C" int vrm_turboquant_decompress(const uint16_t* radius, const uint8_t* 
     set_error("%s: null pointer argument", who);
     return VRM_ERR_ARG;
   }
-  if (tq_rows_ok(padded_dim, bits) && (padded_dim == 64 || N >= kTileMinDecompressRows)) {
+  if (tq_rows_ok(padded_dim, bits) && N >= (padded_dim == 64 ? kTileMinDecompressRows64 : kTileMinDecompressRows)) {
     launch_tq_decompress(rows_args(radius, angles, N, head_dim, padded_dim, bits, false, rotated, signs, angle_lut,
                                    out),
                          reinterpret_cast<hipStream_t>(stream));
