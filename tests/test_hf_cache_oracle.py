@@ -52,3 +52,30 @@ def test_oracle_cache_spill_is_near_lossless_at_8_bits():
     assert cache.layers[0].spills == 1
     assert (got - ref).abs().max() < 2e-2
     assert not torch.equal(got, ref)
+
+
+def test_layer_keeps_one_decode_workspace_per_pass(monkeypatch):
+    """The decode workspaces of a layer do not add up over a generation: two
+    buffers, large enough for any page count, whatever lengths it passed."""
+    from vramancer_amd import tq_pages, turboquant_cache as TC
+    from vramancer_amd.kv_quantizer import KVCacheCompressor
+    from vramancer_amd.paged_attention_cuda import decode_workspace
+
+    B, H, KH, D = 4, 16, 8, 64
+    used = []
+
+    def fake(q, tq_pool, tq_table, tq_lens, comp, res_pool, res_table, res_lens, scale, tq_ws, res_ws, dtype):
+        need = max(decode_workspace(B, H, KH, D, t.shape[1], "cpu").numel() for t in (tq_table, res_table))
+        assert tq_ws.data_ptr() != res_ws.data_ptr() and min(tq_ws.numel(), res_ws.numel()) >= need
+        used.append((tq_ws.data_ptr(), res_ws.data_ptr()))
+        return torch.zeros(q.shape, dtype=dtype)
+
+    monkeypatch.setattr(tq_pages, "paged_attention_decode_residual", fake)
+    layer = TC.TurboQuantLayer(KVCacheCompressor(head_dim=D, bits_per_angle=4), residual_length=128)
+    layer._B, layer._KH, layer._D, layer.device = B, KH, D, torch.device("cpu")
+    layer._rp = 8
+    for n_c in (16, 1000, 5000, 90000):
+        for n_r in range(1, 128, 9):
+            layer._view = (n_c, n_r)
+            assert layer.attend_decode(torch.zeros(B, H, 1, D), 0.125).shape == (B, 1, H, D)
+    assert len(set(used)) == 1 and len(layer._ws) == 2

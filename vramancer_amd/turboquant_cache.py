@@ -273,11 +273,13 @@ class TurboQuantLayer(CacheLayerMixin):
             self._len_last = (n, torch.full((self._B,), n, dtype=torch.int32, device=self.device))
         return self._len_last[1]
 
-    def _workspace(self, kind: str, H: int, pages: int):
-        key = (kind, H, pages)  # one per pass: the merge of a step reads both
+    def _workspace(self, kind: str, H: int):
+        """One buffer per pass, for every length (its size does not depend on
+        the page table's width): the merge of a step reads both."""
+        key = (kind, H)
         ws = self._ws.get(key)
         if ws is None:
-            ws = decode_workspace(self._B, H, self._KH, self._D, pages, self.device)
+            ws = decode_workspace(self._B, H, self._KH, self._D, 1, self.device)
             self._ws[key] = ws
         return ws
 
@@ -294,16 +296,16 @@ class TurboQuantLayer(CacheLayerMixin):
         if n_c and n_r:
             out = tq_pages.paged_attention_decode_residual(
                 q, self._tq_pool, self._table("tq", pj), self._lengths(n_c), self.compressor, self._res_pool,
-                self._table("res", pr), self._lengths(n_r), scale, self._workspace("tq", H, pj),
-                self._workspace("res", H, pr), query.dtype)
+                self._table("res", pr), self._lengths(n_r), scale, self._workspace("tq", H),
+                self._workspace("res", H), query.dtype)
         elif n_c:
             out = tq_pages.paged_attention_decode_turbo(
                 q, self._tq_pool, self._table("tq", pj), self._lengths(n_c), 0, self.compressor, scale=scale,
-                workspace=self._workspace("tq", H, pj),
+                workspace=self._workspace("tq", H),
                 lse=torch.empty((B, H), dtype=torch.float32, device=self.device), qjl=False)
         elif n_r:
             out = paged_attention_decode(q, self._res_pool, self._table("res", pr), self._lengths(n_r), 0,
-                                         scale=scale, workspace=self._workspace("res", H, pr))
+                                         scale=scale, workspace=self._workspace("res", H))
         else:
             out = torch.zeros((B, H, D), dtype=torch.float32, device=self.device)
         return out.to(query.dtype).unsqueeze(1)
