@@ -438,7 +438,8 @@ int vrm_topk_attend(const float* scores, int M, int N, long long ld_scores, int 
  * padded_dim 64 or 128, qjl_dim = padded_dim / 2, bits <= 4 and N <= 32768;
  * VRM_ERR_UNSUPPORTED otherwise.  Angles aligned to 4 bytes, k_signs and
  * workspace to 16.  workspace: >= vrm_turboquant_sparse_attend_workspace_bytes
- * bytes (query features, scores, selection, partial sums).
+ * bytes (query features, scores, selection, partial sums of a pass; large M are
+ * taken in passes over query rows, 256 MB in all).
  */
 size_t vrm_turboquant_sparse_attend_workspace_bytes(int M, int N, int padded_dim, int qjl_dim);
 int vrm_turboquant_sparse_attend(const float* q, int M, const uint16_t* k_radius,

@@ -368,3 +368,12 @@ def test_pass_of_other_calls(lib):
     assert f(8, 40, 8, 128, 16, 64, 2) == 0  # float pools
     assert f(8, 40, 8, 256, 16, 64, 3) == 0 and f(8, 40, 8, 128, 32, 64, 3) == 0  # other shapes
     assert f(8, 40, 7, 128, 16, 64, 3) == -1 and f(0, 40, 8, 128, 16, 64, 3) == -1 and f(8, 40, 8, 128, 16, 64, 9) == -1
+
+
+def test_sparse_attend_workspace_does_not_grow_with_the_query_rows(lib):
+    f = lib.vrm_turboquant_sparse_attend_workspace_bytes
+    for N, pd in ((1, 64), (1000, 128), (32768, 64), (32768, 128)):
+        sizes = [f(M, N, pd, pd // 2) for M in (1, 40, 300, 4096, 65535)]
+        assert sizes == sorted(sizes) and sizes[-1] <= 257 << 20, (N, pd, sizes)
+        one = 4 * (N + pd + pd // 2)  # at least a row's scores and features
+        assert sizes[0] >= one and sizes[1] >= 40 * one

@@ -140,6 +140,21 @@ def test_sparse_v_over_codes_matches_float64(head_dim, bits, M, N, ratio):
     torch.testing.assert_close(comp.sparse_v_attend(q, ck, parts, sparse_v_ratio=ratio), got, atol=0, rtol=0)
 
 
+@pytest.mark.parametrize("head_dim,M,N", [(128, 700, 32768), (64, 2220, 15000)])
+def test_sparse_v_of_many_query_rows(head_dim, M, N):
+    """More query rows than one pass takes (672 and 2208; the last one is short): the rows
+    do not depend on each other, so each comes out as in a call of its own."""
+    _say(f"sparse passes d{head_dim} M{M} N{N}")
+    torch.manual_seed(head_dim)
+    comp = KVCacheCompressor(head_dim, 3).to(DEV)
+    g = torch.Generator().manual_seed(M)
+    ck, cv = (comp.compress(torch.randn(N, head_dim, generator=g).to(DEV), pack=False) for _ in range(2))
+    q = torch.randn(M, head_dim, generator=g).to(DEV)
+    got = comp.sparse_v_attend(q, ck, [cv], sparse_v_ratio=0.05)
+    parts = [comp.sparse_v_attend(q[m:m + 40], ck, [cv], sparse_v_ratio=0.05) for m in range(0, M, 40)]
+    torch.testing.assert_close(got, torch.cat(parts), atol=0, rtol=0)
+
+
 def test_sparse_v_ties_and_values_without_numbers():
     """Equal keys give equal scores, of which the lowest-indexed are kept; a
     value row with an infinite radius reaches the query rows that keep it and

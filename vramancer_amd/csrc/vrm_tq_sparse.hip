@@ -25,6 +25,8 @@
 #include "vrm_tq_scores.h"
 #include "vrm_tq_tile.h"
 
+#include <algorithm>
+
 namespace vrm {
 namespace {
 
@@ -366,16 +368,26 @@ namespace {
 int pv_blocks(int N) { return (N + kPvWaves * kTile - 1) / (kPvWaves * kTile); }
 
 struct SparseWs {
-  size_t scores, rows, sum, part, total;  // byte offsets; the query features come first
+  int rows;                              // query rows of one pass
+  size_t scores, sel, sum, part, total;  // byte offsets; the query features come first
 };
+// Query rows are taken in passes whose scores and partial sums (padded_dim / 64
+// times the scores) stay within kPassBytes, so that the workspace does not grow
+// with M: 4096 rows over 32,768 keys took 1.6 GB, 65,535 rows 26.  Smaller
+// passes leave compute units without a row to select (1024 rows over 32,768
+// keys in one pass 545 us, in passes of 672 rows 560, of 144 740).  A pass is a
+// multiple of the 48 rows that the sum takes at once.
+constexpr size_t kPassBytes = (size_t)256 << 20;
 SparseWs sparse_ws(int M, int N, int padded_dim, int qjl_dim) {
   auto up = [](size_t x) { return (x + 255) / 256 * 256; };
+  const size_t row = ((size_t)N + padded_dim + qjl_dim + (size_t)pv_blocks(N) * (padded_dim + 1)) * sizeof(float);
   SparseWs w{};
-  w.scores = up((size_t)M * (padded_dim + qjl_dim) * sizeof(float));
-  w.rows = w.scores + up((size_t)M * N * sizeof(float));
-  w.sum = w.rows + up((size_t)M * sizeof(TopkRow));
-  w.part = w.sum + up((size_t)pv_blocks(N) * M * sizeof(float));
-  w.total = w.part + (size_t)pv_blocks(N) * M * padded_dim * sizeof(float);
+  w.rows = (int)std::min<size_t>((size_t)M, std::max<size_t>(kPassBytes / row / 48, 1) * 48);
+  w.scores = up((size_t)w.rows * (padded_dim + qjl_dim) * sizeof(float));
+  w.sel = w.scores + up((size_t)w.rows * N * sizeof(float));
+  w.sum = w.sel + up((size_t)w.rows * sizeof(TopkRow));
+  w.part = w.sum + up((size_t)pv_blocks(N) * w.rows * sizeof(float));
+  w.total = w.part + (size_t)pv_blocks(N) * w.rows * padded_dim * sizeof(float);
   return w;
 }
 
@@ -444,18 +456,22 @@ extern "C" int vrm_turboquant_sparse_attend(const float* q, int M, const uint16_
     return VRM_ERR_ARG;
   }
   float* scores = reinterpret_cast<float*>(base + w.scores);
-  TopkRow* rows = reinterpret_cast<TopkRow*>(base + w.rows);
+  TopkRow* rows = reinterpret_cast<TopkRow*>(base + w.sel);
   float* part = reinterpret_cast<float*>(base + w.part);
   float* part_sum = reinterpret_cast<float*>(base + w.sum);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  launch_tq_query(q, M, head_dim, padded_dim, signs, jl, qjl_dim, feat, st);
-  launch_tq_score_tiles(feat, M, keys, N, padded_dim, angle_lut, bits, (float)(sqrt(M_PI / 2.0) / qjl_dim), scale,
-                        scores, st);
-  launch_topk_select(scores, M, N, N, k, rows, st);
   const TqCodes vals{v_radius, v_angles, nullptr, nullptr};
-  if (padded_dim == 64)
-    launch_pv<64>(scores, M, N, rows, vals, angle_lut, bits, head_dim, signs, part, part_sum, out, st);
-  else
-    launch_pv<128>(scores, M, N, rows, vals, angle_lut, bits, head_dim, signs, part, part_sum, out, st);
+  for (int m0 = 0; m0 < M; m0 += w.rows) {
+    const int m = std::min(w.rows, M - m0);
+    launch_tq_query(q + (size_t)m0 * head_dim, m, head_dim, padded_dim, signs, jl, qjl_dim, feat, st);
+    launch_tq_score_tiles(feat, m, keys, N, padded_dim, angle_lut, bits, (float)(sqrt(M_PI / 2.0) / qjl_dim), scale,
+                          scores, st);
+    launch_topk_select(scores, m, N, N, k, rows, st);
+    float* o = out + (size_t)m0 * head_dim;
+    if (padded_dim == 64)
+      launch_pv<64>(scores, m, N, rows, vals, angle_lut, bits, head_dim, signs, part, part_sum, o, st);
+    else
+      launch_pv<128>(scores, m, N, rows, vals, angle_lut, bits, head_dim, signs, part, part_sum, o, st);
+  }
   return launch_status(who);
 }
