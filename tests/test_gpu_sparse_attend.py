@@ -155,6 +155,32 @@ def test_sparse_v_of_many_query_rows(head_dim, M, N):
     torch.testing.assert_close(got, torch.cat(parts), atol=0, rtol=0)
 
 
+def test_sparse_v_of_unaligned_codes():
+    """Rows 1 .. of larger arrays start off the 4-byte alignment that the fused
+    path reads by; the call then decompresses the values, with the same rows
+    kept.  Float32 sums in another order: 1e-5 of each row's largest output."""
+    _say("sparse unaligned")
+    torch.manual_seed(9)
+    comp = KVCacheCompressor(128, 3).to(DEV)
+    g = torch.Generator().manual_seed(9)
+    N = 900
+    ck, cv = (comp.compress(torch.randn(N + 1, 128, generator=g).to(DEV), pack=False) for _ in range(2))
+
+    def rows(c, copy):
+        base = torch.cat(c["angles"], -1) if copy else None
+        dims = [a.shape[1] for a in c["angles"]]
+        ang = list(torch.split(base[1:].clone(), dims, -1)) if copy else [a[1:] for a in c["angles"]]
+        return dict({k: c[k][1:].clone() if copy else c[k][1:] for k in ("radius", "qjl_signs", "qjl_norms")},
+                    angles=ang, shape=(N, 128))
+
+    assert rows(cv, False)["angles"][0].data_ptr() % 4  # 127 bytes a row
+    q = torch.randn(6, 128, generator=g).to(DEV)
+    want = comp.sparse_v_attend(q, rows(ck, True), [rows(cv, True)], sparse_v_ratio=0.1)
+    got = comp.sparse_v_attend(q, rows(ck, False), [rows(cv, False)], sparse_v_ratio=0.1)
+    err = (got - want).abs()
+    assert (err <= 1e-5 * want.abs().amax(-1, keepdim=True)).all(), f"max err {err.max():.3e}"
+
+
 def test_sparse_v_ties_and_values_without_numbers():
     """Equal keys give equal scores, of which the lowest-indexed are kept; a
     value row with an infinite radius reaches the query rows that keep it and
