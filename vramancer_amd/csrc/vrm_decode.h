@@ -320,7 +320,9 @@ constexpr int kMaxUnitsPerWg = 4;  // page-pair counters the LDS layout leaves r
 constexpr int kIdBucketBits = 6;   // a work item's pages are read in 2^6 buckets of ascending page id
 constexpr int kIdBuckets = 1 << kIdBucketBits;
 constexpr size_t kMaxBalancedLds = 64 * 1024;
-constexpr int kSplitMinPages = 96;  // pages from which a sequence is worth two workgroups (split)
+constexpr int kSplitMinPages = 96;  // pages from which a sequence is worth two workgroups (split),
+constexpr int kSplitMean = 3;       // and the multiple of the batch's mean
+__host__ __device__ inline int split_extra(int B) { return (B - 1) / kSplitMean; }
 // LDS one workgroup of the shared-items pass may take on the current device
 // (its 12-wavefront workgroups hold a CU each, so beyond 64 KB costs no
 // occupancy): the device's per-workgroup limit, at most 160 KB.

@@ -824,17 +824,31 @@ __device__ __forceinline__ DecodeArgs kernel_args_afresh() {
   return ai;
 }
 
-// True for a sequence that the batch would wait for: 96 pages or more, and
-// above twice the batch's mean (none in an even batch, none among lengths
+// Sequences that the batch would wait for: kSplitMinPages or more, and above
+// kSplitMean times the batch's mean (none in an even batch, none among lengths
 // spread evenly from an eighth of the longest up: with a lower line those
-// lose, 64 of up to 64 pages 21 -> 31 us at 4/3 of the mean).
-__device__ __forceinline__ bool split_sequence(const DecodeArgs& a, int b) {
+// lose, 64 of up to 64 pages 21 -> 31 us at 4/3 of the mean).  Fewer than one in
+// kSplitMean can be.
+__device__ __forceinline__ bool splits(const DecodeArgs& a, int pages, int total) {
+  return pages >= kSplitMinPages && (long long)pages * a.B > (long long)kSplitMean * total;
+}
+__device__ __forceinline__ int batch_pages(const DecodeArgs& a) {
   const int lane = __lane_id();
   int total = 0;
   for (int c = 0; c < a.B; c += 64) total += c + lane < a.B ? seq_pages(a.ctx_lens[c + lane], a.max_pp) : 0;
-  total = wave_sum_int(total);
-  const int pages = seq_pages(a.ctx_lens[b], a.max_pp);
-  return pages >= kSplitMinPages && (long long)pages * a.B > 3LL * total;
+  return wave_sum_int(total);
+}
+// The k-th of them, or -1.
+__device__ __forceinline__ int split_sequence(const DecodeArgs& a, int k) {
+  const int lane = __lane_id();
+  const int total = batch_pages(a);
+  for (int c = 0; c < a.B; c += 64) {
+    const int pages = c + lane < a.B ? seq_pages(a.ctx_lens[c + lane], a.max_pp) : 0;
+    const unsigned long long m = __ballot(splits(a, pages, total));
+    if (k < __popcll(m)) return c + __builtin_ffsll(__ballot(((m >> lane) & 1) && lane_rank(m) == k)) - 1;
+    k -= __popcll(m);
+  }
+  return -1;
 }
 
 // grid: (work item, unit group), balanced: (sequence, unit group).  ITEMS:
@@ -845,14 +859,13 @@ __device__ __forceinline__ bool split_sequence(const DecodeArgs& a, int b) {
 // merge barrier, so the next piece's page ids and counters overwrite nothing
 // still read.
 //
-// SPLIT (balanced): grid z = 2.  A sequence that the batch would wait for is
-// streamed by two workgroups, one unit each with all wavefronts on it, so that
-// a lone long sequence among short ones costs half its pages' time.  The
-// workgroups of z = 0 have nothing to do for the others and leave at once;
-// they go first, since workgroups dispatched behind the whole batch would
-// start late (one of 256 pages among 47 short ones 32 us, 42 with them last;
-// 64 of 256 pages each 96.5 us, 95.9 without them), and they take the
-// sequences five further on, or at B % 64 == 0 both would queue on one CU.
+// SPLIT (balanced): a grid of one dimension, sequences fastest.  A sequence that
+// the batch would wait for is streamed by two workgroups, one unit each with all
+// wavefronts on it, so that a lone long sequence among short ones costs half
+// its pages' time.  The second workgroups (`extra` per unit pair, as many as
+// there can be such sequences) go first and leave at once if there are fewer:
+// behind the whole batch they would start late (one sequence of 256 pages among
+// 47 short ones 32 us, 42 with them last).
 template <int KIND, int D, bool BALANCED, bool LOADS = false, bool ITEMS = false, int UPW = kUnitsPerWg,
           bool SPLIT = false>
 __global__ void __launch_bounds__(64 * (BALANCED ? kMaxBalancedWaves : kMaxWaves))
@@ -866,11 +879,18 @@ __global__ void __launch_bounds__(64 * (BALANCED ? kMaxBalancedWaves : kMaxWaves
       items = stream_item<KIND, D, BALANCED, LOADS, ITEMS, UPW>(ai, G, item, blockIdx.x);  // 0: no such piece
     }
   } else if constexpr (SPLIT) {
-    const int b = blockIdx.z ? blockIdx.x : (blockIdx.x + 5) % a.B;
-    if (split_sequence(a, b))
-      stream_item<KIND, D, BALANCED, LOADS, ITEMS, 1>(a, G, b, 2 * blockIdx.y + blockIdx.z);
-    else if (blockIdx.z)
-      stream_item<KIND, D, BALANCED, LOADS, ITEMS, UPW>(a, G, b, blockIdx.y);
+    const int extra = split_extra(a.B), pairs = gridDim.x / (a.B + extra);
+    const int id = blockIdx.x;
+    if (id < extra * pairs) {
+      const int b = split_sequence(a, id % extra);
+      if (b >= 0) stream_item<KIND, D, BALANCED, LOADS, ITEMS, 1>(a, G, b, 2 * (id / extra) + 1);
+    } else {
+      const int b = (id - extra * pairs) % a.B, y = (id - extra * pairs) / a.B;
+      if (splits(a, seq_pages(a.ctx_lens[b], a.max_pp), batch_pages(a)))
+        stream_item<KIND, D, BALANCED, LOADS, ITEMS, 1>(a, G, b, 2 * y);
+      else
+        stream_item<KIND, D, BALANCED, LOADS, ITEMS, UPW>(a, G, b, y);
+    }
   } else {
     stream_item<KIND, D, BALANCED, LOADS, ITEMS, UPW>(a, G, blockIdx.x, blockIdx.y);
   }
@@ -1530,10 +1550,13 @@ __global__ void __launch_bounds__(64 * kMaxWaves) decode_stream_q4_kernel(Decode
 // three: at head_dim 112 and 128 the pool's reads run slower with more bytes
 // in flight (32 sequences of 1k-8k tokens, 28 / 4 heads of 128, bf16: 69.2 us
 // with two, 73.8 with three; 64 of 4k, 40 / 8 heads of 112: 182 against 198).
-// Narrower heads are faster with the three or four that fit.
+// Narrower heads are faster with the three or four that fit.  Workgroups of
+// three wavefronts (W = 3, as at 6 kv-heads) get two to a compute unit, six
+// wavefronts: 32 sequences of 4k, 24 / 6 heads of 128, 85.1 us, against 89.3
+// with three of them.
 size_t float_stream_lds(int D, int W) {
   if (D < 112) return 0;
-  const size_t share = (size_t)160 * 1024 / (8 / W);  // 8 wavefronts on a CU's four SIMDs
+  const size_t share = (size_t)160 * 1024 / (8 / W);  // at most 8 wavefronts on a CU's four SIMDs
   return share < 64 * 1024 ? share : 64 * 1024;
 }
 
@@ -1603,8 +1626,8 @@ hipError_t launch_balanced_d(const DecodeArgs& a, int B, int G, hipStream_t st, 
     if (wpu > 1 && (long)B * wgs_y * W > resident) continue;
     if constexpr (!LOADS) {
       if (split && wpu == 6) {
-        hipLaunchKernelGGL((decode_stream_kernel<KIND, D, true, false, false, 2, true>), dim3(B, wgs_y, 2),
-                           dim3(64 * W), lds, st, a, G);
+        hipLaunchKernelGGL((decode_stream_kernel<KIND, D, true, false, false, 2, true>),
+                           dim3((B + split_extra(B)) * wgs_y), dim3(64 * W), lds, st, a, G);
         return hipGetLastError();
       }
     }

@@ -796,7 +796,7 @@ QuantPass quant_pass(int B, int units, int max_pp, int G, int D) {
     if (max_pp <= 200)
       fits = balanced <= items + slack;
     else
-      fits = max_pp <= 300 && balanced <= items * (max_pp <= 256 ? 0.80 : 0.65) * (D >= 96 ? 1.0 : 1.11);
+      fits = max_pp <= 300 && balanced <= items * (max_pp <= 256 ? 0.92 : 0.65) * (D >= 96 ? 1.0 : 1.11);
   } else {
     few = max_pp <= 128;
     const bool half = ((long)B * units - 1) % 512 >= 255;
