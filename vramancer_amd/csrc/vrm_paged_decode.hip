@@ -756,10 +756,10 @@ int check_kind_shape(int kind, int D, int PS, const char* who) {
 // pages; one among ones of a thirtieth to a twelfth).  The lines lie where the
 // worst of these against the fastest pass is least:
 //   up to 256 workgroups balanced follows its cost below; past it, items to
-//     128 workgroups (at 8 sequences of up to 200 pages 0.76 of the shared
-//     rows or less), since the shared rows are the fastest for equal lengths
-//     that fill their rows evenly but two to thirteen times slower than the
-//     others for skewed ones;
+//     128 workgroups (at 8 sequences of up to 200 pages 0.4 to 0.8 of the
+//     shared rows, 1.12 at 160 pages each), since the shared rows are the
+//     fastest for equal lengths that fill their rows evenly but two to thirteen
+//     times slower than the others for skewed ones;
 //   257 to 512, split above 100 pages: up to 300 pages where the cost favours
 //     it by more the longer the table (64 of 256 pages each 96 us against 99;
 //     one of them among short ones 32 us against 42, 51 without the split);

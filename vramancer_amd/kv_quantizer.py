@@ -6,9 +6,10 @@ methods (core/kv_quantizer.py:207-576): the rotation signs and the JL matrix
 are drawn from torch's global RNG in the same order (``randint`` then
 ``randn``), so a compressor built after ``torch.manual_seed(s)`` holds the
 same buffers as the reference's.  Compression, decompression and the
-rotated-space key reconstruction run in gfx950 kernels; the packed format
-(MSB-first bit packing of angles and QJL signs, core/kv_quantizer.py:46-105)
-is produced with tensor ops on the same device.
+rotated-space key reconstruction run in gfx950 kernels, and so does the packed
+format (MSB-first bit packing of angles and QJL signs,
+core/kv_quantizer.py:46-105), which compression writes and decompression reads
+directly at the common settings.
 
 There is no CPU path: CPU tensors raise ``RuntimeError`` and ``force_cpu``
 is rejected (the reference's CPU path is the oracle these kernels are tested
@@ -215,8 +216,10 @@ class KVCacheCompressor(nn.Module):
         """Scores from compressed keys, then the renormalised softmax over the
         top ceil(ratio * seq) scores applied to their values
         (core/kv_quantizer.py:537-562); every step runs in gfx950 kernels.
-        The values are decompressed in one batch; rows of several queries are
-        supported (the reference's sparse branch takes one)."""
+        Up to 32,768 tokens at the common settings the values are summed in the
+        rotated space and never decompressed to memory; other calls decompress
+        them in one batch.  Rows of several queries are supported (the
+        reference's sparse branch takes one)."""
         from .turboquant_cuda import topk_attend
 
         if scale is None:

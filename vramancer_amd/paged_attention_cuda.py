@@ -66,10 +66,11 @@ def decode_workspace(batch: int, num_heads: int, num_kv_heads: int, head_dim: in
     return torch.empty(nbytes, dtype=torch.uint8, device=device)
 
 
-# The balanced decode (one workgroup per sequence and kv-head, partitions
-# merged in LDS; vrm_paged_decode_balanced) replaces the work-item decode when
-# the caller knows the context lengths on the host and they are even: its time
-# follows the longest sequence, the work-item decode's the mean.
+# The balanced decode (one workgroup per sequence and one or two kv-heads,
+# partitions merged in LDS; vrm_paged_decode_balanced) is taken at any length
+# when the caller knows the context lengths on the host and they are even: its
+# time follows the longest sequence, the other passes' the mean.  Without host
+# lengths the library chooses by the call's sizes (vrm_paged_decode_pass).
 BALANCED_MAX_SPREAD = 1.10   # longest context / mean context
 BALANCED_MIN_PAIRS = 128     # sequences x kv-heads: enough workgroups to fill the GPU
 
@@ -149,7 +150,8 @@ def paged_attention_decode(
 
     ``context_lens_host``, when given, must equal ``context_lens``; it only
     selects the kernel (``prefer_balanced``): even batches over int8 / fp8
-    pools take the balanced decode, which needs no workspace.
+    pools take the balanced decode at any length, which needs no workspace.
+    Other calls leave the choice to the library, which goes by their sizes.
     """
     query, page_table, context_lens, scale = _prepare(query, page_table, context_lens, scale)
     _lib.require_cuda(query, kv_pool, page_table, context_lens, kv_scales)

@@ -273,7 +273,9 @@ class CUDATurboQuantOps:
     ):
         """[n_queries, N] scores = q_rot . k_polar + QJL correction
         (core/kv_quantizer.py:502-535), times ``scale``, in two kernels:
-        query rotation and projection, then one wavefront per key."""
+        query rotation and projection, then the product on the matrix cores, 16
+        keys per wavefront (settings or alignments that it does not serve: on
+        the vector units)."""
         import torch
 
         _lib.require_cuda(q)
